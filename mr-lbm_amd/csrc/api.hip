@@ -12,7 +12,9 @@
 #include "../../include/mrlbm.h"
 #include "bc_classes.h"
 #include "context.h"
+#include "init_moments.h"
 #include "kernels.h"
+#include "transfer.h"
 
 using namespace mrlbm;
 
@@ -35,19 +37,12 @@ size_t storage_bytes(int storage) { return storage == MRLBM_STORE_FP32 ? 4 : 2; 
 // host-side storage conversion (round to nearest even; the kernels round
 // stochastically)
 uint16_t to_half(double v) { return __builtin_bit_cast(uint16_t, (_Float16)(float)v); }
-double from_half(uint16_t b) { return (double)(float)__builtin_bit_cast(_Float16, b); }
 uint16_t to_bf16(double v) {
     const float f = (float)v;
     uint32_t u;
     std::memcpy(&u, &f, 4);
     u += 0x7FFFu + ((u >> 16) & 1u);
     return (uint16_t)(u >> 16);
-}
-double from_bf16(uint16_t b) {
-    const uint32_t u = (uint32_t)b << 16;
-    float f;
-    std::memcpy(&f, &u, 4);
-    return (double)f;
 }
 
 }  // namespace mrlbm
@@ -245,51 +240,6 @@ int mrlbm_set_node_types(mrlbm_ctx* c, const uint32_t* types) {
 
 namespace {
 
-// Stored (scaled) moments of one node from unscaled macroscopic fields.
-void node_moments(int q, int mode, double rho0, double rho, double ux, double uy, double uz, double m[10]) {
-    double pxx, pxy, pxz, pyy, pyz, pzz;
-    if (mode == MRLBM_INIT_EQUILIBRIUM) {
-        pxx = ux * ux;
-        pxy = ux * uy;
-        pxz = ux * uz;
-        pyy = uy * uy;
-        pyz = uy * uz;
-        pzz = uz * uz;
-    } else {
-        // f_eq(w_i RHO_0, u), summed over the D3Q19 index subsets and divided
-        // by rho, as src/lbmInitialization.cu:102-130 does for either lattice.
-        static const int CX[19] = {0, 1, -1, 0, 0, 0, 0, 1, -1, 1, -1, 0, 0, 1, -1, 1, -1, 0, 0};
-        static const int CY[19] = {0, 0, 0, 1, -1, 0, 0, 1, -1, 0, 0, 1, -1, -1, 1, 0, 0, 1, -1};
-        static const int CZ[19] = {0, 0, 0, 0, 0, 1, -1, 0, 0, 1, -1, 1, -1, 0, 0, -1, 1, -1, 1};
-        double f[19];
-        const double uu = ux * ux + uy * uy + uz * uz;
-        for (int i = 0; i < 19; i++) {
-            const int cls = i == 0 ? 0 : (i < 7 ? 1 : 2);
-            const double w = q == 19 ? (cls == 0 ? 1.0 / 3 : (cls == 1 ? 1.0 / 18 : 1.0 / 36))
-                                     : (cls == 0 ? 8.0 / 27 : (cls == 1 ? 2.0 / 27 : 1.0 / 54));
-            const double uc3 = 3.0 * (ux * CX[i] + uy * CY[i] + uz * CZ[i]);
-            f[i] = (w * rho0) * ((1.0 - 1.5 * uu) + uc3 * (1.0 + uc3 * 0.5));
-        }
-        const double ir = 1.0 / rho, cs2 = 1.0 / 3.0;
-        pxx = (f[1] + f[2] + f[7] + f[8] + f[9] + f[10] + f[13] + f[14] + f[15] + f[16]) * ir - cs2;
-        pxy = ((f[7] + f[8]) - (f[13] + f[14])) * ir;
-        pxz = ((f[9] + f[10]) - (f[15] + f[16])) * ir;
-        pyy = (f[3] + f[4] + f[7] + f[8] + f[11] + f[12] + f[13] + f[14] + f[17] + f[18]) * ir - cs2;
-        pyz = ((f[11] + f[12]) - (f[17] + f[18])) * ir;
-        pzz = (f[5] + f[6] + f[9] + f[10] + f[11] + f[12] + f[15] + f[16] + f[17] + f[18]) * ir - cs2;
-    }
-    m[0] = rho - rho0;
-    m[1] = 3.0 * ux;
-    m[2] = 3.0 * uy;
-    m[3] = 3.0 * uz;
-    m[4] = 4.5 * pxx;
-    m[5] = 9.0 * pxy;
-    m[6] = 9.0 * pxz;
-    m[7] = 4.5 * pyy;
-    m[8] = 9.0 * pyz;
-    m[9] = 4.5 * pzz;
-}
-
 // One stored moment (index m, stored convention) -> its storage word
 uint32_t encode_value(const mrlbm_ctx* c, int m, double x) {
     const double v = x * c->mscale[m];
@@ -300,44 +250,6 @@ uint32_t encode_value(const mrlbm_ctx* c, int m, double x) {
         return u;
     }
     return c->p.storage == MRLBM_STORE_FP16 ? to_half(v) : to_bf16(v);
-}
-
-// Moments (block layout, doubles, stored convention) -> storage bytes
-std::vector<char> encode_block(const mrlbm_ctx* c, const std::vector<double>& blk) {
-    const size_t sb = storage_bytes(c->p.storage);
-    std::vector<char> raw(blk.size() * sb);
-    const size_t T = c->T;
-    for (size_t j = 0; j < blk.size(); j++) {
-        const uint32_t u = encode_value(c, (int)((j / T) % 10), blk[j]);
-        if (sb == 4) {
-            std::memcpy(&raw[j * 4], &u, 4);
-        } else {
-            const uint16_t h = (uint16_t)u;
-            std::memcpy(&raw[j * 2], &h, 2);
-        }
-    }
-    return raw;
-}
-
-std::vector<double> decode_block(const mrlbm_ctx* c, const std::vector<char>& raw) {
-    const size_t sb = storage_bytes(c->p.storage);
-    std::vector<double> blk(raw.size() / sb);
-    const size_t T = c->T;
-    for (size_t j = 0; j < blk.size(); j++) {
-        const int m = (int)((j / T) % 10);
-        double v;
-        if (c->p.storage == MRLBM_STORE_FP32) {
-            float f;
-            std::memcpy(&f, &raw[j * 4], 4);
-            v = f;
-        } else {
-            uint16_t h;
-            std::memcpy(&h, &raw[j * 2], 2);
-            v = c->p.storage == MRLBM_STORE_FP16 ? from_half(h) : from_bf16(h);
-        }
-        blk[j] = v * (double)c->mrscale[m];
-    }
-    return blk;
 }
 
 // Both ghost sets from the stored moments; the lattice restarts at step 0.
@@ -359,30 +271,10 @@ int ghosts_from_moments(mrlbm_ctx* c) {
     return MRLBM_OK;
 }
 
-int upload_and_ghosts(mrlbm_ctx* c, const std::vector<double>& blk) {
-    HIPCHK(hipSetDevice(c->p.device));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    const std::vector<char> raw = encode_block(c, blk);
-    HIPCHK(hipMemcpy(c->d_mom, raw.data(), raw.size(), hipMemcpyHostToDevice));
-    return ghosts_from_moments(c);
-}
-
-template <typename F>
-int init_with(mrlbm_ctx* c, int mode, F&& field) {
+int check_mode(int mode) {
     if (mode != MRLBM_INIT_EQUILIBRIUM && mode != MRLBM_INIT_REFERENCE)
         return fail(MRLBM_EINVAL, "unknown second-moment mode %d", mode);
-    std::vector<double> blk(c->N * 10);
-    const int nx = c->p.nx, ny = c->p.ny, nz = c->p.nz;
-    for (int z = 0; z < nz; z++)
-        for (int y = 0; y < ny; y++)
-            for (int x = 0; x < nx; x++) {
-                double r, ux, uy, uz, m[10];
-                field(x, y, z, r, ux, uy, uz);
-                if (!(r > 0)) return fail(MRLBM_EINVAL, "non-positive density at (%d,%d,%d)", x, y, z);
-                node_moments(c->p.q, mode, c->p.rho0, r, ux, uy, uz, m);
-                for (int k = 0; k < 10; k++) blk[c->mom_index(x, y, z, k)] = m[k];
-            }
-    return upload_and_ghosts(c, blk);
+    return MRLBM_OK;
 }
 
 }  // namespace
@@ -392,20 +284,15 @@ extern "C" {
 int mrlbm_init_fields(mrlbm_ctx* c, const double* rho, const double* ux, const double* uy, const double* uz,
                       int mode) {
     if (!c || !rho || !ux || !uy || !uz) return fail(MRLBM_EINVAL, "null argument");
-    const size_t nx = c->p.nx, ny = c->p.ny;
-    return init_with(c, mode, [&](int x, int y, int z, double& r, double& a, double& b, double& d) {
-        const size_t j = x + nx * (y + ny * z);
-        r = rho[j];
-        a = ux[j];
-        b = uy[j];
-        d = uz[j];
-    });
+    int rc = check_mode(mode);
+    if (!rc) rc = write_fields_linear(c, mode, rho, ux, uy, uz);
+    return rc ? rc : ghosts_from_moments(c);
 }
 
 int mrlbm_init_uniform(mrlbm_ctx* c, double rho, double ux, double uy, double uz, int mode) {
     if (!c) return fail(MRLBM_EINVAL, "null context");
-    if (mode != MRLBM_INIT_EQUILIBRIUM && mode != MRLBM_INIT_REFERENCE)
-        return fail(MRLBM_EINVAL, "unknown second-moment mode %d", mode);
+    int rc = check_mode(mode);
+    if (rc) return rc;
     if (!(rho > 0)) return fail(MRLBM_EINVAL, "non-positive density");
     // one node's stored moments, encoded once and filled on the device
     double m[10];
@@ -413,23 +300,15 @@ int mrlbm_init_uniform(mrlbm_ctx* c, double rho, double ux, double uy, double uz
     uint32_t enc[10];
     for (int k = 0; k < 10; k++) enc[k] = encode_value(c, k, m[k]);
     HIPCHK(hipSetDevice(c->p.device));
-    int rc = fill_uniform_moments(c, enc);
-    if (rc) return rc;
+    if ((rc = fill_uniform_moments(c, enc))) return rc;
     return ghosts_from_moments(c);
 }
 
 int mrlbm_init_taylor_green(mrlbm_ctx* c, double u0, int mode) {
     if (!c) return fail(MRLBM_EINVAL, "null context");
-    // cases/taylorGreen/flow_initialization.inc:1-4 with L = N/(2 pi)
-    const double kx = 2.0 * M_PI / c->p.nx, ky = 2.0 * M_PI / c->p.ny, kz = 2.0 * M_PI / c->p.nz;
-    const double rho0 = c->p.rho0;
-    return init_with(c, mode, [&](int x, int y, int z, double& r, double& a, double& b, double& d) {
-        r = rho0 + (3.0 / 16.0) * rho0 * u0 * u0 * (std::cos(2 * kx * x) + std::cos(2 * ky * y)) *
-                       (std::cos(2 * kz * z) + 2.0);
-        a = u0 * std::sin(kx * x) * std::cos(ky * y) * std::cos(kz * z);
-        b = -u0 * std::cos(kx * x) * std::sin(ky * y) * std::cos(kz * z);
-        d = 0.0;
-    });
+    int rc = check_mode(mode);
+    if (!rc) rc = write_taylor_green(c, u0, mode);
+    return rc ? rc : ghosts_from_moments(c);
 }
 
 static int do_steps(mrlbm_ctx* c, int nsteps) {
@@ -498,30 +377,13 @@ int mrlbm_synchronize(mrlbm_ctx* c) {
 
 int mrlbm_read_moments(mrlbm_ctx* c, double* out) {
     if (!c || !out) return fail(MRLBM_EINVAL, "null argument");
-    HIPCHK(hipSetDevice(c->p.device));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    std::vector<char> raw(c->N * 10 * storage_bytes(c->p.storage));
-    HIPCHK(hipMemcpy(raw.data(), c->d_mom, raw.size(), hipMemcpyDeviceToHost));
-    const std::vector<double> blk = decode_block(c, raw);
-    const int nx = c->p.nx, ny = c->p.ny, nz = c->p.nz;
-    for (int k = 0; k < 10; k++)
-        for (int z = 0; z < nz; z++)
-            for (int y = 0; y < ny; y++)
-                for (int x = 0; x < nx; x++)
-                    out[(size_t)k * c->N + x + (size_t)nx * (y + (size_t)ny * z)] = blk[c->mom_index(x, y, z, k)];
-    return MRLBM_OK;
+    return read_moments_linear(c, out);
 }
 
 int mrlbm_write_moments(mrlbm_ctx* c, const double* in) {
     if (!c || !in) return fail(MRLBM_EINVAL, "null argument");
-    std::vector<double> blk(c->N * 10);
-    const int nx = c->p.nx, ny = c->p.ny, nz = c->p.nz;
-    for (int k = 0; k < 10; k++)
-        for (int z = 0; z < nz; z++)
-            for (int y = 0; y < ny; y++)
-                for (int x = 0; x < nx; x++)
-                    blk[c->mom_index(x, y, z, k)] = in[(size_t)k * c->N + x + (size_t)nx * (y + (size_t)ny * z)];
-    return upload_and_ghosts(c, blk);
+    const int rc = write_moments_linear(c, in);
+    return rc ? rc : ghosts_from_moments(c);
 }
 
 int mrlbm_reduce_checked(mrlbm_ctx* c, double* mass, double* ke, int64_t* nonfinite) {

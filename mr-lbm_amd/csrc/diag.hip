@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "context.h"
+#include "transfer.h"
 
 using namespace mrlbm;
 
@@ -219,11 +220,8 @@ int mrlbm_mean_flow_accumulate(mrlbm_ctx* c) {
 int mrlbm_mean_flow_read(mrlbm_ctx* c, double* out, int64_t* count) {
     if (!c || !out || !count) return fail(MRLBM_EINVAL, "null argument");
     if (!c->d_mean || c->mean_count == 0) return fail(MRLBM_ESTATE, "no mean-flow samples accumulated");
-    HIPCHK(hipSetDevice(c->p.device));
-    HIPCHK(hipMemcpyAsync(out, c->d_mean, sizeof(double) * 4 * c->N, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    const double inv = 1.0 / (double)c->mean_count;
-    for (size_t j = 0; j < 4 * c->N; j++) out[j] *= inv;
+    const int rc = read_scaled(c, c->d_mean, 4 * c->N, 1.0 / (double)c->mean_count, out);
+    if (rc) return rc;
     *count = c->mean_count;
     return MRLBM_OK;
 }
