@@ -30,7 +30,7 @@ void hermite(int i, double h[6]) {
     h[5] = CZ[i] * CZ[i] - t;
 }
 const double COEF[6] = {1, 2, 2, 1, 2, 1};
-constexpr int BC_REC = 72;  // floats per class record (lattice.h BC_STRIDE)
+constexpr int BC_REC = 64;  // floats per class record (lattice.h BC_STRIDE)
 }  // namespace
 
 uint32_t known_mask(int q, uint32_t octants) {
@@ -129,7 +129,8 @@ bool class_record(int q, uint32_t octants, double omega, const double u[3], floa
     rec[1] = (float)u[0];
     rec[2] = (float)u[1];
     rec[3] = (float)u[2];
-    for (int k = 0; k < 49; k++) rec[4 + k] = (float)ainv[k];
+    for (int k = 0; k < 7; k++)
+        for (int j = 0; j < 6; j++) rec[19 + 6 * k + j] = (float)ainv[7 * k + 1 + j];
     // rest-state split of the right-hand side (populations travel
     // as f_i - w_i RHO_0): W_K, c = sum_K w_i H_i / W_K, and the rest
     // solution y_rest = A^-1 (1, c), d0 = W_K y_rest,0 - 1
@@ -147,10 +148,10 @@ bool class_record(int q, uint32_t octants, double omega, const double u[3], floa
         yrest[k] = 0;
         for (int j = 0; j < 7; j++) yrest[k] += ainv[7 * k + j] * brest[j];
     }
-    rec[53] = (float)wk;
-    for (int j = 0; j < 6; j++) rec[54 + j] = (float)brest[1 + j];
-    rec[60] = (float)(wk * yrest[0] - 1.0);
-    for (int k = 0; k < 7; k++) rec[61 + k] = (float)yrest[k];
+    rec[4] = (float)wk;
+    for (int j = 0; j < 6; j++) rec[5 + j] = (float)brest[1 + j];
+    rec[11] = (float)(wk * yrest[0] - 1.0);
+    for (int k = 0; k < 7; k++) rec[12 + k] = (float)yrest[k];
     return true;
 }
 

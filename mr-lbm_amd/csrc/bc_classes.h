@@ -35,7 +35,7 @@ int closure_lattice(int q, uint32_t octants);
 
 struct BcClassTable {
     std::vector<uint32_t> keys;      // node-type key (octants | kind | velocity index) per class, index 1..
-    std::vector<float> table;        // 72 floats per class (lattice.h BC_STRIDE; class 0 unused)
+    std::vector<float> table;        // 64 floats per class (lattice.h BC_STRIDE; class 0 unused)
     std::vector<uint8_t> class_of;   // per node in the caller's x-fastest order
     bool has_bc = false, has_solid = false;
 };

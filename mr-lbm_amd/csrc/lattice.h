@@ -323,11 +323,13 @@ __device__ __forceinline__ void bulk_moments(const float* g, float rho0, Node& n
 // Boundary-condition class record (device table, BC_STRIDE floats per class).
 //   [0]       bit mask of known populations (bit i set = population i known)
 //   [1..3]    wall velocity (unscaled)
-//   [4..52]   A^-1, inverse of the 7x7 moment-matching system, row-major
-//   [53]      W_K = sum_{i in K} w_i
-//   [54..59]  c_k = sum_{i in K} w_i H_i,k / W_K   (k = xx, xy, xz, yy, yz, zz)
-//   [60]      d0  = W_K y_rest,0 - 1
-//   [61..67]  y_rest = A^-1 (1, c)  (the solution for the rest state)
+//   [4]       W_K = sum_{i in K} w_i
+//   [5..10]   c_k = sum_{i in K} w_i H_i,k / W_K   (k = xx, xy, xz, yy, yz, zz)
+//   [11]      d0  = W_K y_rest,0 - 1
+//   [12..18]  y_rest = A^-1 (1, c)  (the solution for the rest state)
+//   [19..60]  A^-1, inverse of the 7x7 moment-matching system, row-major,
+//             without its first column (the right-hand side (0, db) skips it)
+// A record is 256 bytes, two lines of the vector L1.
 // The system (one per class, built on the host in FP64) is the one whose
 // closed-form solutions are the reference's generated bc_definition.inc
 // formulas: with P = rho m,
@@ -335,7 +337,7 @@ __device__ __forceinline__ void bulk_moments(const float* g, float rho0, Node& n
 //   sum_{i in K} f^R_i(rho, u_w, m) H_i,ab                     = rho_I m_I,ab
 // where K is the known set, rho_I = sum_K f_i and m_I = sum_K f_i H_i / rho_I;
 // x = (rho, P) = rho_I A^-1 (1, m_I).
-constexpr int BC_STRIDE = 72;
+constexpr int BC_STRIDE = 64;
 
 // Moment-based boundary condition at a node of class `c`, from the sums of
 // its known streamed deviations (f_i = w_i RHO_0 + g_i; moment_sums over g
@@ -345,42 +347,65 @@ constexpr int BC_STRIDE = 72;
 // the FP32 arithmetic forms is a small deviation. Outputs unscaled rho, u, m
 // exactly as a bc_definition.inc fragment does (src/mlbm.cu:456-461); the
 // caller scales.
+//
+// The record comes as a type with get<K>(): entry K.
 template <typename P>
-__device__ __forceinline__ void bc_from_sums(P c, const Sums& S, float rho0, Node& n) {
+struct PointerRecord {  // per-lane record
+    P p;
+    template <int K>
+    __device__ __forceinline__ float get() const {
+        return p[K];
+    }
+};
+// Record shared by the wave's boundary nodes: lane l holds entries l % 16 of
+// four runs of 16, and an instruction's DPP operand broadcasts the entry it
+// needs within each row of 16 lanes. All lanes must be active.
+struct RowRecord {
+    float v[4];
+    template <int K>
+    __device__ __forceinline__ float get() const {
+        return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v[K / 16]), 0x150 + K % 16, 0xF, 0xF, true));
+    }
+};
+
+template <typename R>
+__device__ __forceinline__ void bc_from_sums(const R& c, const Sums& S, float rho0, Node& n) {
     const float r = S.r, sxx = S.sxx, syy = S.syy, szz = S.szz, sxy = S.sxy, sxz = S.sxz, syz = S.syz;
-    const float rI = rho0 * c[53] + r;
+    const float rI = rho0 * c.template get<4>() + r;
     const float inv = __builtin_amdgcn_rcpf(rI);  // v_rcp_f32 (1 ulp): the BC moments' rounding level
     const float r3 = r * (1.0f / 3.0f);
     float db[6];
-    db[0] = ((sxx - r3) - c[54] * r) * inv;
-    db[1] = (sxy - c[55] * r) * inv;
-    db[2] = (sxz - c[56] * r) * inv;
-    db[3] = ((syy - r3) - c[57] * r) * inv;
-    db[4] = (syz - c[58] * r) * inv;
-    db[5] = ((szz - r3) - c[59] * r) * inv;
+    db[0] = ((sxx - r3) - c.template get<5>() * r) * inv;
+    db[1] = (sxy - c.template get<6>() * r) * inv;
+    db[2] = (sxz - c.template get<7>() * r) * inv;
+    db[3] = ((syy - r3) - c.template get<8>() * r) * inv;
+    db[4] = (syz - c.template get<9>() * r) * inv;
+    db[5] = ((szz - r3) - c.template get<10>() * r) * inv;
     float dy[7];
-#pragma unroll
-    for (int k = 0; k < 7; k++) {
-        float acc = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 6; j++) acc = acc + c[4 + 7 * k + 1 + j] * db[j];
+    static_for<7>([&](auto K) {
+        constexpr int k = decltype(K)::value;
+        float acc = c.template get<19 + 6 * k>() * db[0];
+        static_for<5>([&](auto J) {
+            constexpr int j = decltype(J)::value + 1;
+            acc = acc + c.template get<19 + 6 * k + j>() * db[j];
+        });
         dy[k] = acc;
-    }
-    const float y0 = c[61] + dy[0];
+    });
+    const float y0 = c.template get<12>() + dy[0];
     const float iy0 = __builtin_amdgcn_rcpf(y0);
     // rho - RHO_0 = rho_I y0 - RHO_0 = RHO_0 d0 + r y_rest,0 + rho_I dy0
-    n.drho = (rho0 * c[60] + r * c[61]) + rI * dy[0];
+    n.drho = (rho0 * c.template get<11>() + r * c.template get<12>()) + rI * dy[0];
     n.rho = rho0 + n.drho;
     n.inv = __builtin_amdgcn_rcpf(n.rho);
-    n.ux = c[1];
-    n.uy = c[2];
-    n.uz = c[3];
-    n.mxx = (c[62] + dy[1]) * iy0;
-    n.mxy = (c[63] + dy[2]) * iy0;
-    n.mxz = (c[64] + dy[3]) * iy0;
-    n.myy = (c[65] + dy[4]) * iy0;
-    n.myz = (c[66] + dy[5]) * iy0;
-    n.mzz = (c[67] + dy[6]) * iy0;
+    n.ux = c.template get<1>();
+    n.uy = c.template get<2>();
+    n.uz = c.template get<3>();
+    n.mxx = (c.template get<13>() + dy[1]) * iy0;
+    n.mxy = (c.template get<14>() + dy[2]) * iy0;
+    n.mxz = (c.template get<15>() + dy[3]) * iy0;
+    n.myy = (c.template get<16>() + dy[4]) * iy0;
+    n.myz = (c.template get<17>() + dy[5]) * iy0;
+    n.mzz = (c.template get<18>() + dy[6]) * iy0;
 }
 
 // Zero the populations a boundary node does not know (bit i of `known`
@@ -399,7 +424,7 @@ __device__ __forceinline__ void bc_solve(P c, float* g, float rho0, Node& n) {
     known_only<Q>(__float_as_uint(c[0]), g);
     Sums S;
     moment_sums<Q>(g, S);
-    bc_from_sums(c, S, rho0, n);
+    bc_from_sums(PointerRecord<P>{c}, S, rho0, n);
 }
 
 // Scale unscaled u, m to the stored convention (src/mlbm.cu:500-509),

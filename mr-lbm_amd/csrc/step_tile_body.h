@@ -285,6 +285,50 @@ __device__ __forceinline__ void tile_update(const StepArgs& a, float* gout, uint
     const uint32_t cls = in.cls;
     const bool solid = HAS_BC && (cls == 255u);
 
+    // Class records of the wave's boundary nodes. They depend on the class
+    // byte, and caches are cold at the start of a launch, so a record read
+    // at the solve costs a second trip to memory; and read per lane it costs
+    // 16 four-dword loads that all fetch the same bytes (about 270 cycles of
+    // the CU's address unit per wave). A wave mostly holds one or two classes
+    // (a wall, a wall and its edge): it fetches their records here, one float
+    // per lane, and the solve broadcasts the entries by DPP. Waves of more
+    // classes (voxelised surfaces, cavity corners) keep the per-lane reads:
+    // a broadcast solve per class costs all lanes' arithmetic each time
+    // (three or four classes that way: 32^3 cavity 7.1 -> 9.0 us per step).
+    // D3Q27 fetches the second record at the solve (with both held ahead its
+    // body spills at 64 VGPRs: 256x128x128 duct 92.8 -> 95.7 us).
+    // Before, all waves read per lane at the solve: FP32 cavities 32^3 7.97
+    // -> 7.06 us, 64^3 9.26 -> 8.37 us, 256^3 301 -> 290.5 us; BF16 duct
+    // 200x72x104 with 6 spheres 26.7 -> 24.8 us; D3Q27 duct 256x128x128
+    // 102.6 -> 92.8 us (with one launch per step, below).
+    const bool bcn = HAS_BC && cls != 0u && cls != 255u;
+    const auto rec = gptr(a.bc) + (size_t)cls * BC_STRIDE;
+    constexpr bool TWO_AHEAD = Q == 19;
+    uint32_t known = ~0u, uc0 = 0, uc1 = 0;
+    bool many = false;
+    RowRecord rr{}, rr1{};
+    auto row_record = [&](uint32_t uc, RowRecord& r) {
+        const auto p = gptr(a.bc) + (size_t)uc * BC_STRIDE;
+        for (int k = 0; k < 4; k++) r.v[k] = (p + 16 * k)[(uint32_t)lane % 16];
+    };
+    const uint64_t bcw = HAS_BC ? __builtin_amdgcn_ballot_w64(bcn) : 0;
+    if constexpr (HAS_BC) {
+        if (bcw != 0) {  // uniform: waves without boundary nodes skip
+            if (bcn) known = __float_as_uint(rec[0]);
+            uc0 = uc1 = (uint32_t)__builtin_amdgcn_readlane((int)cls, __builtin_ctzll(bcw));
+            uint64_t rest = bcw & ~__builtin_amdgcn_ballot_w64(cls == uc0);
+            if (rest != 0) {
+                uc1 = (uint32_t)__builtin_amdgcn_readlane((int)cls, __builtin_ctzll(rest));
+                rest &= ~__builtin_amdgcn_ballot_w64(cls == uc1);
+            }
+            many = rest != 0;
+            if (!many) {
+                row_record(uc0, rr);
+                if (TWO_AHEAD && uc1 != uc0) row_record(uc1, rr1);
+            }
+        }
+    }
+
     // FP16: the reconstruction reads the fetched binary16 words directly
     // (recon_terms_f16); FP32, BF16: decoded moments
     constexpr bool F16 = S == 1;
@@ -374,20 +418,33 @@ __device__ __forceinline__ void tile_update(const StepArgs& a, float* gout, uint
     if constexpr (HAS_BC) {
         // boundary nodes: one pass of moment sums shared with the bulk nodes
         // of the wave, over their known populations only (the others zeroed)
-        const bool bcn = cls != 0u && cls != 255u;
-        const uint64_t bcw = __builtin_amdgcn_ballot_w64(bcn);
-        if (bcw != 0) {  // uniform: waves without boundary nodes skip
-            uint32_t known = ~0u;
-            if (bcn) known = __float_as_uint(gptr(a.bc)[(size_t)cls * BC_STRIDE]);
-            known_only<Q>(known, g);
-        }
+        if (bcw != 0) known_only<Q>(known, g);
         Sums sums;
         moment_sums<Q>(g, sums);
-        if (bcn) {
-            bc_from_sums(gptr(a.bc) + (size_t)cls * BC_STRIDE, sums, a.rho0, m);
-            scale_moments(m, SU, SM);
-        } else {
-            bulk_from_sums(sums, a.rho0, m, SU, SM);
+        bulk_from_sums(sums, a.rho0, m, SU, SM);
+        if (bcw != 0) {
+            if (!many) {
+#pragma unroll 1
+                for (uint32_t uc = uc0;; uc = uc1) {
+                    Node b;
+                    bc_from_sums(rr, sums, a.rho0, b);
+                    scale_moments(b, SU, SM);
+                    // every lane computes it (the broadcasts need the whole
+                    // wave): keep the arithmetic out of the branch below
+                    asm("" : "+v"(b.drho), "+v"(b.rho), "+v"(b.inv), "+v"(b.mxx), "+v"(b.mxy), "+v"(b.mxz), "+v"(b.myy),
+                        "+v"(b.myz), "+v"(b.mzz));
+                    asm("" : "+v"(b.ux), "+v"(b.uy), "+v"(b.uz));
+                    if (cls == uc) m = b;
+                    if (uc == uc1) break;
+                    if constexpr (TWO_AHEAD)
+                        rr = rr1;
+                    else
+                        row_record(uc1, rr);
+                }
+            } else if (bcn) {
+                bc_from_sums(PointerRecord<decltype(rec)>{rec}, sums, a.rho0, m);
+                scale_moments(m, SU, SM);
+            }
         }
     } else {
         bulk_moments<Q>(g, a.rho0, m, SU, SM);
@@ -449,23 +506,15 @@ constexpr int lds_waves_per_simd() {
     return w > 8 ? 8 : (w < 1 ? 1 : w);
 }
 
-// Register budget of a step body: the bulk body, the FP32 D3Q19 boundary
-// bodies with x rows of at most 16 nodes and the 16-bit D3Q19 boundary
-// bodies with 8-node rows (~64 VGPRs at 8 waves per SIMD) take the waves the
-// LDS allows; the D3Q27 boundary bodies with rows of at most 16 nodes at most
-// 6 waves (80 VGPRs; at 8 waves they spill); other boundary bodies keep the
-// compiler's choice (a tighter budget spills VGPRs to memory). The ranged
-// batched kernel also holds the next item's fetch: its boundary bodies and
-// its D3Q27 bodies keep the compiler's choice.
+// Register budget of a step body: the waves the LDS allows (64 VGPRs at 8
+// waves per SIMD). Exceptions, where that budget spills VGPRs to memory and
+// the compiler's choice is kept: boundary bodies with x rows of more than 16
+// nodes, and in the ranged batched kernel, which also holds the next item's
+// fetch, the boundary and the D3Q27 bodies.
 template <int Q, int BX, int BY, int BZ, bool HAS_BC, int S, bool RANGED = false>
 constexpr int step_body_waves() {
     constexpr int w = lds_waves_per_simd<Q, BX, BY, BZ, HAS_BC>();
-    if constexpr (HAS_BC) {
-        if constexpr (RANGED) return 1;
-        if constexpr (Q == 19 && BX <= (S == 0 ? 16 : 8)) return w;
-        if constexpr (Q == 27 && BX <= 16) return w > 6 ? 6 : w;
-        return 1;
-    }
+    if constexpr (HAS_BC) return (RANGED || BX > 16) ? 1 : w;
     return (RANGED && Q == 27) ? 1 : w;
 }
 
@@ -549,14 +598,15 @@ void k_step_batch1(const InstArgs* __restrict__ tab, const uint32_t* __restrict_
 }
 
 // Both bodies in one launch, where they run at the same occupancy (the same
-// LDS size and register budget: D3Q19 8x8x8 in every storage format, FP32
-// 16x8x8): blocks [0, nbulk) take all-bulk tiles with the bulk body, the
-// others tiles with boundary or solid nodes. One launch per step instead of
-// two: the second launch's ramp-up and the first one's tail overlap.
+// register budget and workgroups per CU: 8x8x8, 16x8x4 and 16x8x8 in every
+// storage format): blocks [0, nbulk) take all-bulk tiles with the bulk body,
+// the others tiles with boundary or solid nodes. One launch per step instead
+// of two: the second launch's ramp-up and the first one's tail overlap
+// (D3Q27 duct 128x64x64 BF16 with 5 spheres 22.9 -> 16.3 us per step together
+// with the row records; 512x256x256 FP16 622 -> 615 us).
 template <int Q, int BX, int BY, int BZ, int S>
 constexpr bool mixed_launch() {
-    return step_body_waves<Q, BX, BY, BZ, false, S>() == step_body_waves<Q, BX, BY, BZ, true, S>() &&
-           sizeof(TileLds<Q, BX, BY, BZ, false>) == sizeof(TileLds<Q, BX, BY, BZ, true>);
+    return step_body_waves<Q, BX, BY, BZ, false, S>() == step_body_waves<Q, BX, BY, BZ, true, S>();
 }
 
 template <int Q, int BX, int BY, int BZ, int S>
