@@ -164,12 +164,13 @@ __host__ __device__ constexpr int window_rows(int face) {
     return r < bv ? r : bv;
 }
 
-// Split rows [vlo, vhi] of a face into windows; calls emit(w0, vlo', vhi').
+// Split rows [vlo, vhi] of a face into windows that start at multiples of
+// `rows` (a divisor of the face's rows); calls emit(w0, vlo', vhi').
 template <typename F>
-constexpr void for_windows(int bv, int rows, int vlo, int vhi, F&& emit) {
+constexpr void for_windows(int rows, int vlo, int vhi, F&& emit) {
     int w = vlo;
     while (w <= vhi) {
-        const int w0 = w + rows <= bv ? w : bv - rows;
+        const int w0 = w - w % rows;
         const int hi = (w0 + rows - 1) < vhi ? (w0 + rows - 1) : vhi;
         emit(w0, w, hi);
         w = hi + 1;
@@ -212,11 +213,10 @@ constexpr int incoming_chunks_of(int i, Chunk* out) {
             }
         }
         if (hi[ua] < lo[ua] || hi[va] < lo[va]) continue;
-        const int bv = G::B[va];
         // a single fixed row is read alone (a taller window would fetch
         // lines no cell needs)
         const int rows = mv[va] ? window_rows<BX, BY, BZ>(face) : 1;
-        for_windows(bv, rows, lo[va], hi[va], [&](int w0, int vlo, int vhi) {
+        for_windows(rows, lo[va], hi[va], [&](int w0, int vlo, int vhi) {
             if (out) {
                 Chunk ch{};
                 ch.face = face;
@@ -275,7 +275,7 @@ constexpr int outgoing_chunks_impl(Chunk* out) {
         const int rows = window_rows<BX, BY, BZ>(face);
         for (int s = 0; s < QF; s++) {
             const int i = face_pop(face, s);
-            for_windows(bv, rows, 0, bv - 1, [&](int w0, int vlo, int vhi) {
+            for_windows(rows, 0, bv - 1, [&](int w0, int vlo, int vhi) {
                 if (out) {
                     Chunk ch{};
                     ch.face = face;
@@ -320,6 +320,69 @@ template <int Q, int BX, int BY, int BZ>
 struct ChunkTables {
     static constexpr auto in = incoming_chunks<Q, BX, BY, BZ>();
     static constexpr auto out = outgoing_chunks<Q, BX, BY, BZ>();
+};
+
+// Which wave moves which chunk. The chunks of one face window that come from
+// the tile across that face (all its slots: contiguous planes of one owner)
+// go to one wave, so that they share one address; the short runs from edge
+// and corner neighbours, each with an owner of its own, fill the waves that
+// hold the fewest, those without a face window first.
+template <int Q, int BX, int BY, int BZ>
+struct InPlan {
+    static constexpr int NW = BX * BY * BZ / 64;
+    static constexpr int NIN = n_incoming_chunks<Q, BX, BY, BZ>();
+    int n[NW] = {};
+    int id[NW][NIN] = {};
+    constexpr int rmax() const {
+        int m = 0;
+        for (int w = 0; w < NW; w++) m = n[w] > m ? n[w] : m;
+        return m;
+    }
+    constexpr InPlan() {
+        constexpr auto in = incoming_chunks<Q, BX, BY, BZ>();
+        bool done[NIN] = {};
+        int w = 0;
+        for (int k = 0; k < NIN; k++) {
+            if (done[k] || !direct(in[k])) continue;
+            for (int j = k; j < NIN; j++)
+                if (!done[j] && direct(in[j]) && in[j].face == in[k].face && in[j].w0 == in[k].w0) {
+                    id[w][n[w]++] = j;
+                    done[j] = true;
+                }
+            w = (w + 1) % NW;
+        }
+        for (int k = 0; k < NIN; k++) {
+            if (done[k]) continue;
+            int best = NW - 1;
+            for (int v = NW - 2; v >= 0; v--)
+                if (n[v] < n[best]) best = v;
+            id[best][n[best]++] = k;
+        }
+    }
+    static constexpr bool direct(const Chunk& c) { return (c.dx != 0) + (c.dy != 0) + (c.dz != 0) == 1; }
+};
+template <int Q, int BX, int BY, int BZ>
+inline constexpr InPlan<Q, BX, BY, BZ> in_plan_v{};
+
+// Outgoing units: one window of one face, all its slots (the chunks of a
+// face lie slot by slot, window by window).
+template <int Q, int BX, int BY, int BZ>
+struct OutUnits {
+    static constexpr int QF = VS<Q>::QF;
+    static constexpr int N = n_outgoing_chunks<Q, BX, BY, BZ>() / QF;
+    __host__ __device__ static constexpr int windows(int face) {
+        return face_bv<BX, BY, BZ>(face) / window_rows<BX, BY, BZ>(face);
+    }
+    // chunk of slot s of unit u
+    __host__ __device__ static constexpr int chunk(int u, int s) {
+        int first = 0, face = 0;
+        while (u >= windows(face)) {
+            u -= windows(face);
+            first += windows(face) * QF;
+            face++;
+        }
+        return first + s * windows(face) + u;
+    }
 };
 
 }  // namespace mrlbm

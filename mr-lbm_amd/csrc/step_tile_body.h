@@ -70,6 +70,14 @@ __device__ __forceinline__ bool chunk_cell(int lane, int& u, int& r) {
     return (Bu * c.rows >= 64 || lane < Bu * c.rows) && u >= c.ulo && u <= c.uhi && v >= c.vlo && v <= c.vhi;
 }
 
+// Terms that the populations leaving through a face read.
+template <int Q>
+constexpr uint32_t face_uses(int face) {
+    uint32_t m = 0;
+    for (int s = 0; s < VS<Q>::QF; s++) m |= recon_uses<Q>(face_pop(face, s));
+    return m;
+}
+
 template <int Q, int BX, int BY, int BZ, int K>
 __device__ __forceinline__ void halo_put(int lane, float v, float* s) {
     constexpr Chunk c = ChunkTables<Q, BX, BY, BZ>::in[K];
@@ -77,13 +85,23 @@ __device__ __forceinline__ void halo_put(int lane, float v, float* s) {
     if (chunk_cell<Q, BX, BY, BZ, true, K>(lane, u, r)) s[c.lds0 + u * c.su + r * c.sv] = v;
 }
 
-// Outgoing chunk K: the lane's face node evaluates the chunk's population
-// from the reconstruction terms the node staged in LDS (term k of the node
-// at base nb is s[k * E + nb]) and writes it to the ghost plane.
-template <int Q, int BX, int BY, int BZ, bool HAS_BC, int K>
+// Outgoing unit U, one window of one face: the lane's face node evaluates
+// the face's QF populations from the reconstruction terms the node staged in
+// LDS (term k of the node at base nb is s[k * E + nb]) and writes them to
+// the slots' planes of the ghost face. One wave does all slots of a window,
+// so the terms they share are read once (10 LDS reads instead of 23 for the
+// five populations of a D3Q19 face) and the planes share one address. With
+// the incoming chunks grouped the same way (InPlan), per wave of FP16 8x8x8:
+// VALU 304 -> 290, scalar 208 -> 151, LDS 54 -> 48 instructions. Per step:
+// FP16 256x192x160 95.7 -> 92.6 us, FP32 256^3 284.4 -> 278.4, FP16 D3Q27
+// 512x256x256 614 -> 575, 64^3 cavity 8.40 -> 8.05.
+template <int Q, int BX, int BY, int BZ, bool HAS_BC, int U>
 __device__ __forceinline__ void halo_store(const StepArgs& a, float* gout, int lane, int tile, int bx, int by,
                                            int bz, const float* s, const uint8_t* s_cls) {
-    constexpr Chunk c = ChunkTables<Q, BX, BY, BZ>::out[K];
+    using CT = ChunkTables<Q, BX, BY, BZ>;
+    using OU = OutUnits<Q, BX, BY, BZ>;
+    constexpr int K0 = OU::chunk(U, 0);
+    constexpr Chunk c = CT::out[K0];
     constexpr int QF = VS<Q>::QF;
     constexpr int Bu = face_bu<BX, BY, BZ>(c.face);
     constexpr int Bv = face_bv<BX, BY, BZ>(c.face);
@@ -99,9 +117,9 @@ __device__ __forceinline__ void halo_store(const StepArgs& a, float* gout, int l
     if constexpr (c.face == 5) skip = a.wall_z && bz == a.ntz - 1;
     if (skip) return;
     const auto dst = gptr(ghost_face<BX, BY, BZ, QF>(gout, c.face, a.ntiles)) +
-                     (size_t)(Bu * Bv) * (c.slot + QF * (size_t)tile) + Bu * c.w0;
+                     (size_t)(Bu * Bv) * (QF * (size_t)tile) + Bu * c.w0;
     int u, r;
-    if (chunk_cell<Q, BX, BY, BZ, false, K>(lane, u, r)) {
+    if (chunk_cell<Q, BX, BY, BZ, false, K0>(lane, u, r)) {
         if constexpr (HAS_BC) {
             // node of the face cell; solid nodes write no ghost values
             constexpr int ax = c.face / 2;
@@ -113,13 +131,16 @@ __device__ __forceinline__ void halo_store(const StepArgs& a, float* gout, int l
             if (s_cls[nx + BX * (ny + BY * nz)] == 255u) return;
         }
         const int nb = c.lds0 + u * c.su + r * c.sv;  // staged-term base of the face node
-        constexpr uint32_t uses = recon_uses<Q>(c.pop);
         Recon t;
         static_for<Recon::N>([&](auto KK) {
             constexpr int k = decltype(KK)::value;
-            t.at(k) = ((uses >> k) & 1u) ? s[k * G::E + nb] : 0.0f;
+            t.at(k) = ((face_uses<Q>(c.face) >> k) & 1u) ? s[k * G::E + nb] : 0.0f;
         });
-        dst[(uint32_t)lane] = recon_pop<Q, c.pop>(t);
+        static_for<QF>([&](auto SS) {
+            constexpr int slot = decltype(SS)::value;
+            constexpr int pop = CT::out[OU::chunk(U, slot)].pop;
+            dst[(uint32_t)lane + Bu * Bv * slot] = recon_pop<Q, pop>(t);
+        });
     }
 }
 
@@ -151,8 +172,7 @@ struct TileLds {
 template <int Q, int BX, int BY, int BZ, int S>
 struct TileIn {
     static constexpr int NW = BX * BY * BZ / 64;
-    static constexpr int NIN = (int)ChunkTables<Q, BX, BY, BZ>::in.size();
-    static constexpr int RMAX = (NIN + NW - 1) / NW;
+    static constexpr int RMAX = in_plan_v<Q, BX, BY, BZ>.rmax();
     typename Fetched<S>::T m[10];
     float h[RMAX];
     uint32_t cls;
@@ -197,7 +217,6 @@ __device__ __forceinline__ void tile_fetch(const StepArgs& a, const float* gin, 
                                            TileIn<Q, BX, BY, BZ, S>& in) {
     constexpr int T = BX * BY * BZ;
     constexpr int NW = T / 64;
-    constexpr int NIN = TileIn<Q, BX, BY, BZ, S>::NIN;
     const int t = thread_index<T>();
     const int lane = t % 64;
     const int w = __builtin_amdgcn_readfirstlane(t / 64);
@@ -242,16 +261,16 @@ __device__ __forceinline__ void tile_fetch(const StepArgs& a, const float* gin, 
             in.m[k] = (typename Fetched<S>::T)__builtin_nontemporal_load(plane);
         }
     }
-    // wave W owns incoming chunks W, W + NW, ...; every wave fills all
-    // RMAX slots (zeros past its last chunk) so that no slot index depends
-    // on the wave (a wave-dependent index would move the array to scratch)
+    // every wave fills all RMAX slots (zeros past its last chunk) so that no
+    // slot index depends on the wave (a wave-dependent index would move the
+    // array to scratch)
     constexpr int RMAX = TileIn<Q, BX, BY, BZ, S>::RMAX;
     dispatch<NW>(w, [&](auto WW) {
         constexpr int W = decltype(WW)::value;
         static_for<RMAX>([&](auto RR) {
             constexpr int r = decltype(RR)::value;
-            if constexpr (W + NW * r < NIN)
-                in.h[r] = halo_fetch<Q, BX, BY, BZ, W + NW * r>(gin, lane, nb);
+            if constexpr (r < in_plan_v<Q, BX, BY, BZ>.n[W])
+                in.h[r] = halo_fetch<Q, BX, BY, BZ, in_plan_v<Q, BX, BY, BZ>.id[W][r]>(gin, lane, nb);
             else
                 in.h[r] = 0.0f;
         });
@@ -269,8 +288,7 @@ __device__ __forceinline__ void tile_update(const StepArgs& a, float* gout, uint
     constexpr int NW = T / 64;
     using G = HaloGeom<BX, BY, BZ>;
     constexpr int E = G::E;
-    constexpr int NIN = TileIn<Q, BX, BY, BZ, S>::NIN;
-    constexpr int NOUT = (int)ChunkTables<Q, BX, BY, BZ>::out.size();
+    constexpr int NOUT = OutUnits<Q, BX, BY, BZ>::N;
     float* s = L.s;
     uint8_t* s_cls = L.cls();
 
@@ -341,16 +359,19 @@ __device__ __forceinline__ void tile_update(const StepArgs& a, float* gout, uint
     auto halo_phase = [&](auto PP) {
         dispatch<NW>(w, [&](auto WW) {
             constexpr int W = decltype(WW)::value;
-            constexpr int R = (NIN - W + NW - 1) / NW;
-            static_for<R>([&](auto RR) {
+            static_for<in_plan_v<Q, BX, BY, BZ>.n[W]>([&](auto RR) {
                 constexpr int r = decltype(RR)::value;
-                constexpr int K = W + NW * r;
+                constexpr int K = in_plan_v<Q, BX, BY, BZ>.id[W][r];
                 if constexpr (P::phase(ChunkTables<Q, BX, BY, BZ>::in[K].pop) == decltype(PP)::value)
                     halo_put<Q, BX, BY, BZ, K>(lane, in.h[r], s);
             });
         });
     };
-    halo_phase(std::integral_constant<int, 0>());
+    // phase 0's halo goes to LDS after the tile's own populations, so that
+    // these do not wait for the ghost chunks; D3Q27, short of registers, frees
+    // the chunks first (512x256x256 FP16 577 us, after the populations 593)
+    constexpr bool PUT_LATE = Q == 19;
+    if constexpr (!PUT_LATE) halo_phase(std::integral_constant<int, 0>());
 
     // population arrays: node base per (x extent, y extent) pair of the
     // arrays, so every access is a base register plus an immediate
@@ -386,10 +407,7 @@ __device__ __forceinline__ void tile_update(const StepArgs& a, float* gout, uint
     // reads and the second phase's writes)
     static_for<PH>([&](auto PP) {
         constexpr int ph = decltype(PP)::value;
-        if constexpr (ph > 0) {
-            __syncthreads();
-            halo_phase(PP);
-        }
+        if constexpr (ph > 0) __syncthreads();
         static_for<Q - 1>([&](auto I) {
             constexpr int i = decltype(I)::value + 1;
             if constexpr (!P::x_only(i) && P::phase(i) == ph) {
@@ -397,6 +415,7 @@ __device__ __forceinline__ void tile_update(const StepArgs& a, float* gout, uint
                 s[pbase(I) + wo] = g[i];
             }
         });
+        if constexpr (PUT_LATE || ph > 0) halo_phase(PP);
         if constexpr (ph == 0) ahead();
         __syncthreads();
         static_for<Q - 1>([&](auto I) {
