@@ -63,6 +63,7 @@ int refresh(mrlbm_batch* b) {
     if (n > 4095) return fail(MRLBM_EINVAL, "a batch holds at most 4095 lattices");
     std::vector<InstArgs> tab(n);
     std::vector<uint32_t> work, bc_work;
+    double bytes = 0;
     for (int i = 0; i < n; i++) {
         mrlbm_ctx* c = b->members[i];
         if (!c->initialised) return fail(MRLBM_ESTATE, "batch member %d is not initialised", i);
@@ -75,6 +76,7 @@ int refresh(mrlbm_batch* b) {
         ia.step0 = (uint32_t)c->step;
         ia.has_bc = c->has_bc ? 1 : 0;
         tab[i] = ia;
+        bytes += c->bytes_per_lu() * (double)c->N;
         const std::vector<uint8_t>* flags = nullptr;
         int rc = tile_flags(c, &flags);
         if (rc) return rc;
@@ -82,6 +84,10 @@ int refresh(mrlbm_batch* b) {
             ((*flags)[t] ? bc_work : work).push_back(((uint32_t)i << 20) | (uint32_t)t);
     }
     const int nbulk = (int)work.size();
+    if (b->grid_limit <= 0) {  // with a grid limit each workgroup walks neighbouring items
+        group_by_xcd(work.data(), work.size(), bytes);
+        group_by_xcd(bc_work.data(), bc_work.size(), bytes);
+    }
     work.insert(work.end(), bc_work.begin(), bc_work.end());
     HIPCHK(hipSetDevice(b->device));
     HIPCHK(hipStreamSynchronize(b->stream));
@@ -250,6 +256,7 @@ int mrlbm_batch_remove(mrlbm_batch* b, mrlbm_ctx* c) {
 
 int mrlbm_batch_set_grid(mrlbm_batch* b, int max_blocks) {
     if (!b || max_blocks < 0) return fail(MRLBM_EINVAL, "bad argument");
+    if ((b->grid_limit > 0) != (max_blocks > 0)) b->dirty = true;  // the item order differs
     b->grid_limit = max_blocks;
     drop_graph(b);
     return MRLBM_OK;

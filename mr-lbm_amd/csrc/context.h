@@ -112,6 +112,7 @@ struct mrlbm_ctx {
         }
         a.step = (uint32_t)step;
         a.seed = p.seed;
+        a.group_end = mrlbm::xcd_group_end((size_t)ntiles, bytes_per_lu() * (double)N);
         return a;
     }
     double bytes_per_lu() const {
@@ -135,6 +136,9 @@ int tile_flags(mrlbm_ctx* c, const std::vector<uint8_t>** out);
 // Device list of the lattice's tiles, all-bulk ones first (n_bulk_tiles),
 // for the split bulk/boundary launches of a lattice with boundary nodes.
 int build_tile_list(mrlbm_ctx* c);
+
+// A launch list's entries in the order of xcd_grouped.
+void group_by_xcd(uint32_t* list, size_t n, double bytes_per_step);
 
 // The stream a batch launches on (members' work is ordered on it).
 hipStream_t batch_stream(const mrlbm_batch* b);

@@ -86,6 +86,32 @@ __device__ __forceinline__ uint32_t sr_bits(uint32_t node, uint32_t step, uint32
     return x;
 }
 
+// Tile order over the XCDs. Workgroup b runs on XCD b % 8, so tiles that lie
+// side by side, which read some of the same ghost lines (one as a face
+// neighbour, the other across an edge), run on different XCDs with L2s of
+// their own. Regrouped, each XCD takes XCD_GROUP consecutive tiles at a time
+// (out of every 8 * XCD_GROUP). Measured per step, before -> after, groups of
+// 32: FP32 96x72x80 15.3 -> 13.2 us, 192x160x128 64.3 -> 62.5; FP16 128^3 27.4
+// -> 26.6, 256x192x160 89.2 -> 88.4; FP32 D3Q27 256x128x128 90.2 -> 84.7, and
+// larger groups give that back from 64 on (192x160x128 62.9 at 64, 63.6 at 128).
+// Steps that move more than the caches hold run better spread evenly over the
+// memory channels: FP32 256^3 278.5 -> 282 us, D3Q27 512x256x256 747 -> 753 us
+// in groups of 32; 256x256x256 FP16 (1.2 GB) and 64x512x256 FP32 (0.9 GB,
+// 131 -> 128 us) mark where the line lies.
+constexpr uint32_t XCD_GROUP = 32;
+constexpr double XCD_GROUP_MAX_BYTES = 1.1e9;  // per step, of the lattice or batch
+// Position that workgroup b takes, of which [0, end) are regrouped.
+__host__ __device__ inline uint32_t xcd_grouped(uint32_t b, uint32_t end) {
+    constexpr uint32_t span = 8 * XCD_GROUP;
+    if (b >= end) return b;
+    return b - b % span + (b % 8) * XCD_GROUP + b / 8 % XCD_GROUP;
+}
+// Regrouped positions of a launch over n tiles that moves `bytes` per step.
+inline uint32_t xcd_group_end(size_t n, double bytes) {
+    constexpr size_t span = 8 * XCD_GROUP;
+    return bytes < XCD_GROUP_MAX_BYTES ? (uint32_t)(n / span * span) : 0u;
+}
+
 // Arguments of one lattice step. Ghost faces: index 0 X_0, 1 X_1, 2 Y_0,
 // 3 Y_1, 4 Z_0, 5 Z_1. `gin` is read (previous step's outgoing
 // populations), `gout` is written; the host swaps them after each step as
@@ -107,6 +133,7 @@ struct StepArgs {
     float mrscale[10];       // inverse scale
     uint32_t step;           // time step being computed (stochastic rounding key)
     uint32_t seed;           // lattice seed (stochastic rounding key)
+    uint32_t group_end;      // tiles taken in XCD groups (xcd_grouped), from tile 0
 };
 
 // Ghost-plane indices of the reference layout with runtime tile shape

@@ -205,6 +205,12 @@ int tile_flags(mrlbm_ctx* c, const std::vector<uint8_t>** out) {
     return MRLBM_OK;
 }
 
+void group_by_xcd(uint32_t* list, size_t n, double bytes_per_step) {
+    const uint32_t end = xcd_group_end(n, bytes_per_step);
+    const std::vector<uint32_t> in(list, list + end);
+    for (uint32_t b = 0; b < end; b++) list[b] = in[xcd_grouped(b, end)];
+}
+
 int build_tile_list(mrlbm_ctx* c) {
     c->n_bulk_tiles = c->ntiles;
     if (!c->has_bc || !c->d_cls) return MRLBM_OK;
@@ -218,6 +224,9 @@ int build_tile_list(mrlbm_ctx* c) {
     c->n_bulk_tiles = (int)list.size();
     for (int t = 0; t < c->ntiles; t++)
         if ((*flags)[t]) list.push_back((uint32_t)t);
+    const double bytes = c->bytes_per_lu() * (double)c->N;
+    group_by_xcd(list.data(), (size_t)c->n_bulk_tiles, bytes);
+    group_by_xcd(list.data() + c->n_bulk_tiles, (size_t)(c->ntiles - c->n_bulk_tiles), bytes);
     if (!c->d_tiles) HIPCHK(hipMalloc((void**)&c->d_tiles, sizeof(uint32_t) * c->ntiles));
     HIPCHK(hipMemcpyAsync(c->d_tiles, list.data(), sizeof(uint32_t) * c->ntiles, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));

@@ -537,7 +537,8 @@ constexpr int step_body_waves() {
     return (RANGED && Q == 27) ? 1 : w;
 }
 
-// Tile step: block b updates tile list[b] (tile b when `list` is null), one
+// Tile step: block b updates tile list[b] (without a list, the tile
+// xcd_grouped gives it), one
 // tile per block: workgroup turnover hides the load latency better than a
 // resident grid walking tiles with a prefetch of the next one (measured on
 // 256^3), and the single-tile body holds fewer scalar registers. For
@@ -547,7 +548,8 @@ template <int Q, int BX, int BY, int BZ, bool HAS_BC, int S>
 __global__ __launch_bounds__(BX* BY* BZ) __attribute__((amdgpu_waves_per_eu(step_body_waves<Q, BX, BY, BZ, HAS_BC, S>())))
 void k_step_tile(StepArgs a, const uint32_t* __restrict__ list) {
     __shared__ TileLds<Q, BX, BY, BZ, HAS_BC> L;
-    const int tile = list ? (int)__builtin_amdgcn_readfirstlane(list[blockIdx.x]) : (int)blockIdx.x;
+    const int tile = list ? (int)__builtin_amdgcn_readfirstlane(list[blockIdx.x])
+                          : (int)xcd_grouped(blockIdx.x, a.group_end);
     TileIn<Q, BX, BY, BZ, S> in;
     tile_fetch<Q, BX, BY, BZ, HAS_BC, S>(a, a.gin, tile, in);
     tile_update<Q, BX, BY, BZ, HAS_BC, S>(a, a.gout, a.step, tile, L, in, []() {});
