@@ -14,6 +14,7 @@
 #include "context.h"
 #include "init_moments.h"
 #include "kernels.h"
+#include "linear.h"
 #include "transfer.h"
 
 using namespace mrlbm;
@@ -45,6 +46,16 @@ uint16_t to_bf16(double v) {
     return (uint16_t)(u >> 16);
 }
 
+int small_buffer(mrlbm_ctx* c) {
+    if (c->h_small) return MRLBM_OK;
+    const hipError_t e = hipHostMalloc((void**)&c->h_small, SMALL_BYTES, hipHostMallocDefault);
+    if (e != hipSuccess) {
+        c->h_small = nullptr;
+        return fail(MRLBM_ENOMEM, "pinned result buffer: %s", hipGetErrorString(e));
+    }
+    return MRLBM_OK;
+}
+
 }  // namespace mrlbm
 
 extern "C" {
@@ -64,7 +75,7 @@ int mrlbm_destroy(mrlbm_ctx* c) {
     for (int s = 0; s < 2; s++)
         hipFree(c->d_gbase[s]);
     hipFree(c->d_partial);
-    hipFree(c->d_red);
+    if (c->h_small) hipHostFree(c->h_small);
     hipFree(c->d_uprev);
     if (c->ev0) hipEventDestroy(c->ev0);
     if (c->ev1) hipEventDestroy(c->ev1);
@@ -182,9 +193,7 @@ int mrlbm_create(const mrlbm_params* pp, mrlbm_ctx** out) {
             o += c->face_elems[f];
         }
     }
-    c->red_blocks = 1024;
-    if ((rc = alloc((void**)&c->d_partial, sizeof(double) * 3 * c->red_blocks)) ||
-        (rc = alloc((void**)&c->d_red, sizeof(double) * 4))) {
+    if ((rc = alloc((void**)&c->d_partial, sizeof(double) * 10 * RED_BLOCKS_MAX))) {
         mrlbm_destroy(c);
         return rc;
     }
@@ -389,10 +398,10 @@ int mrlbm_write_moments(mrlbm_ctx* c, const double* in) {
 int mrlbm_reduce_checked(mrlbm_ctx* c, double* mass, double* ke, int64_t* nonfinite) {
     if (!c || !mass || !ke || !nonfinite) return fail(MRLBM_EINVAL, "null argument");
     HIPCHK(hipSetDevice(c->p.device));
+    if (int rc = small_buffer(c)) return rc;
+    double* const h = (double*)c->h_small;
     HIPCHK(launch_reduce(c->p.storage, c->d_mom, c->ntiles, c->T, (float)c->p.rho0, c->mrscale[0], c->mrscale[1],
-                         c->d_partial, c->red_blocks, c->d_red, c->stream, (double)c->N));
-    double h[3];
-    HIPCHK(hipMemcpyAsync(h, c->d_red, sizeof h, hipMemcpyDeviceToHost, c->stream));
+                         c->d_partial, h, c->stream, (double)c->N));
     HIPCHK(hipStreamSynchronize(c->stream));
     *mass = h[0];
     *ke = h[1];
@@ -419,10 +428,10 @@ int mrlbm_velocity_residual(mrlbm_ctx* c, double* residual) {
         c->device_bytes += (double)bytes;
         HIPCHK(hipMemsetAsync(c->d_uprev, 0, bytes, c->stream));
     }
-    HIPCHK(launch_residual(c->p.storage, c->d_mom, c->d_uprev, c->ntiles, c->T, c->mrscale[1], c->d_partial,
-                           c->red_blocks, c->d_red, c->stream));
-    double h[3];
-    HIPCHK(hipMemcpyAsync(h, c->d_red, sizeof h, hipMemcpyDeviceToHost, c->stream));
+    if (int rc = small_buffer(c)) return rc;
+    double* const h = (double*)c->h_small;
+    HIPCHK(launch_residual(c->p.storage, c->d_mom, c->d_uprev, c->ntiles, c->T, c->mrscale[1], c->d_partial, h,
+                           c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     *residual = first ? -1.0 : (h[1] > 0.0 ? std::sqrt(h[0] / h[1]) : (h[0] > 0.0 ? INFINITY : 0.0));
     return MRLBM_OK;

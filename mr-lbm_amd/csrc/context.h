@@ -42,9 +42,8 @@ struct mrlbm_ctx {
     bool has_bc = false, has_solid = false, initialised = false;
     int n_classes = 0;
     double bc_vel[4][3] = {};
-    double* d_partial = nullptr;
-    double* d_red = nullptr;
-    int red_blocks = 0;
+    double* d_partial = nullptr;  // partial sums: 1024 records of at most ten values
+    char* h_small = nullptr;      // pinned: results of sums, sample points and values (SMALL_BYTES, on first use)
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     double device_bytes = 0;
     mrlbm_batch* batch = nullptr;  // batch this lattice is stepped in (its stream is then the batch's)
@@ -142,6 +141,11 @@ void group_by_xcd(uint32_t* list, size_t n, double bytes_per_step);
 
 // The stream a batch launches on (members' work is ordered on it).
 hipStream_t batch_stream(const mrlbm_batch* b);
+
+// The context's small pinned buffer, which kernels read and write in place: a
+// result is on the host when the stream is idle, without a copy of its own.
+constexpr size_t SMALL_BYTES = 64 * 1024;
+int small_buffer(mrlbm_ctx* c);
 
 // Device address of the allocation-free reduction's scratch array on
 // `device` (which must be current), looked up on the first call for that

@@ -317,8 +317,8 @@ struct GpuDevice {
         for (int i = 0; i < n_checked; i++) {
             const mrlbm_ctx* c = active[i].ctx;
             const hipError_t he = launch_reduce(c->p.storage, c->d_mom, c->ntiles, c->T, (float)c->p.rho0,
-                                                c->mrscale[0], c->mrscale[1], c->d_partial, c->red_blocks,
-                                                d_health + 3 * i, s);
+                                                c->mrscale[0], c->mrscale[1], c->d_partial, d_health + 3 * i, s,
+                                                (double)c->N);
             if (he != hipSuccess) return fail(MRLBM_EHIP, "health reduction: %s", hipGetErrorString(he));
         }
         if (n_checked &&

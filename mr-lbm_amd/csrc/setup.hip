@@ -291,7 +291,7 @@ int mrlbm_set_geometry(mrlbm_ctx* c, const uint8_t* solid, int nspheres, const d
             first = 0;
         }
     }
-    uint32_t* d_occ = (uint32_t*)c->d_partial;  // reduction scratch, 2 * red_blocks doubles
+    uint32_t* d_occ = (uint32_t*)c->d_partial;  // reduction scratch
     k_zero_words<<<1, 64, 0, c->stream>>>(d_occ, 8);
     k_classify<<<blocks_for(c->N, 256), 256, 0, c->stream>>>(e, d_solid, c->d_cls, d_occ);
     HIPCHK(hipGetLastError());

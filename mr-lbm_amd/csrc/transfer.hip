@@ -24,6 +24,7 @@
 
 #include "context.h"
 #include "init_moments.h"
+#include "linear.h"
 #include "transfer.h"
 
 using namespace mrlbm;
@@ -137,82 +138,6 @@ int pump(mrlbm_ctx* c, size_t chunks, Launch&& launch, Take&& take) {
     if (e != hipSuccess) return fail(MRLBM_EHIP, "field transfer: %s", hipGetErrorString(e));
     return MRLBM_OK;
 }
-
-// x-fastest order in groups of four nodes along x (every tile is a multiple
-// of four nodes wide, so a group is one 16- or 8-byte run of a moment plane)
-// and the block layout. Tile extents are powers of two.
-struct Linear {
-    FastDiv by_nx4, by_ny;
-    uint32_t nx4, ny, ntx, nty, T;
-    uint32_t groups;  // per plane
-    int lx, ly, lz;   // log2 of the tile extents
-    float scale[10], rscale[10];
-    // element of moment 0 of the group's first node; moment m lies m T further
-    __device__ __forceinline__ size_t node(uint32_t group) const {
-        const uint32_t row = by_nx4.div(group), z = by_ny.div(row);
-        const uint32_t x = 4 * (group - row * nx4), y = row - z * ny;
-        const uint32_t tile = (x >> lx) + ntx * ((y >> ly) + nty * (z >> lz));
-        const uint32_t t = (x & ((1u << lx) - 1)) + ((y & ((1u << ly) - 1)) << lx) + ((z & ((1u << lz) - 1)) << (lx + ly));
-        return (size_t)tile * 10 * T + t;
-    }
-};
-
-int log2_of(int v) {
-    int l = 0;
-    while ((1 << l) < v) l++;
-    return l;
-}
-
-Linear linear_of(const mrlbm_ctx* c) {
-    Linear L{};
-    L.nx4 = (uint32_t)c->p.nx / 4;
-    L.ny = (uint32_t)c->p.ny;
-    L.by_nx4 = make_fastdiv(L.nx4);
-    L.by_ny = make_fastdiv(L.ny);
-    L.ntx = (uint32_t)c->ntx;
-    L.nty = (uint32_t)c->nty;
-    L.T = (uint32_t)c->T;
-    L.groups = (uint32_t)(c->N / 4);
-    L.lx = log2_of(c->bx);
-    L.ly = log2_of(c->by);
-    L.lz = log2_of(c->bz);
-    for (int m = 0; m < 10; m++) {
-        L.scale[m] = c->mscale[m];
-        L.rscale[m] = c->mrscale[m];
-    }
-    return L;
-}
-
-// Storage word of a stored moment, rounded to nearest even (through FP32),
-// and back, as the host encodes single values (to_half, to_bf16).
-template <int S> struct Word;
-template <> struct Word<0> {
-    using T = uint32_t;
-    typedef uint32_t __attribute__((ext_vector_type(4))) V;
-    __device__ static float dec(uint32_t w, float) { return __uint_as_float(w); }
-    __device__ static uint32_t enc(double v, float s) { return __float_as_uint((float)(v * (double)s)); }
-};
-template <> struct Word<1> {
-    using T = uint16_t;
-    typedef uint16_t __attribute__((ext_vector_type(4))) V;
-    __device__ static float dec(uint16_t w, float rs) { return (float)__builtin_bit_cast(_Float16, w) * rs; }
-    __device__ static uint16_t enc(double v, float s) {
-        return __builtin_bit_cast(uint16_t, (_Float16)(float)(v * (double)s));
-    }
-};
-template <> struct Word<2> {
-    using T = uint16_t;
-    typedef uint16_t __attribute__((ext_vector_type(4))) V;
-    __device__ static float dec(uint16_t w, float) { return __uint_as_float((uint32_t)w << 16); }
-    __device__ static uint16_t enc(double v, float s) {
-        uint32_t u = __float_as_uint((float)(v * (double)s));
-        u += 0x7FFFu + ((u >> 16) & 1u);
-        return (uint16_t)(u >> 16);
-    }
-};
-
-typedef float __attribute__((ext_vector_type(4))) f32x4;
-typedef double __attribute__((ext_vector_type(4))) f64x4;
 
 // Moment plane and group of group `i` of a chunk that starts at group j0 of
 // plane k0 (a chunk of a small lattice spans planes).
