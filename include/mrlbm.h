@@ -144,6 +144,11 @@ int mrlbm_synchronize(mrlbm_ctx* ctx);
  * 9mxz, 4.5myy, 9myz, 4.5mzz (src/arrayIndex.h:8-17,186). */
 int mrlbm_read_moments(mrlbm_ctx* ctx, double* out10n);
 
+/* Density and velocity as doubles, x-fastest, 4 planes of N values: the stored
+ * rho-RHO_0 plus rho0, and the stored 3u over 3 (the fields that saveMacr
+ * writes, src/saveData.cu:7-260), without the second moments. */
+int mrlbm_read_macroscopic(mrlbm_ctx* ctx, double rho0, double* out4n);
+
 /* Overwrite the stored moments (same format) and rebuild both ghost sets
  * from them, as gpuInitialization_pop does. */
 int mrlbm_write_moments(mrlbm_ctx* ctx, const double* in10n);

@@ -81,6 +81,7 @@ int mrlbm_destroy(mrlbm_ctx* c) {
     if (c->ev1) hipEventDestroy(c->ev1);
     if (c->stream) hipStreamDestroy(c->stream);
     delete c;
+    count_lattices(-1);
     return MRLBM_OK;
 }
 
@@ -138,6 +139,7 @@ int mrlbm_create(const mrlbm_params* pp, mrlbm_ctx** out) {
     if (int rc0 = noalloc_scratch_setup(p.device, nullptr)) return rc0;
 
     mrlbm_ctx* c = new mrlbm_ctx();
+    count_lattices(1);
     c->p = p;
     if (c->p.rho0 == 0.0) c->p.rho0 = 1.0;
     c->p.bx = c->bx = bx;
@@ -387,6 +389,11 @@ int mrlbm_synchronize(mrlbm_ctx* c) {
 int mrlbm_read_moments(mrlbm_ctx* c, double* out) {
     if (!c || !out) return fail(MRLBM_EINVAL, "null argument");
     return read_moments_linear(c, out);
+}
+
+int mrlbm_read_macroscopic(mrlbm_ctx* c, double rho0, double* out) {
+    if (!c || !out) return fail(MRLBM_EINVAL, "null argument");
+    return read_macroscopic_linear(c, rho0, out);
 }
 
 int mrlbm_write_moments(mrlbm_ctx* c, const double* in) {

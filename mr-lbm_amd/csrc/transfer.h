@@ -8,8 +8,14 @@ struct mrlbm_ctx;
 
 namespace mrlbm {
 
+// Lattices that live (+1, -1): the process's pinned transfer slots are kept
+// while there are any.
+void count_lattices(int d);
+
 // Stored moments decoded into out[k * N + x + NX (y + NY z)].
 int read_moments_linear(mrlbm_ctx* c, double* out);
+// rho0 + (rho - RHO_0), ux, uy, uz: four such planes.
+int read_macroscopic_linear(mrlbm_ctx* c, double rho0, double* out);
 // Stored moments from the same layout.
 int write_moments_linear(mrlbm_ctx* c, const double* in);
 // Stored moments from density and velocity fields; refuses a non-positive

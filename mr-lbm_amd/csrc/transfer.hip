@@ -17,6 +17,7 @@
 #include <atomic>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <system_error>
 #include <thread>
@@ -66,26 +67,79 @@ void run_workers(int n, F&& f) {
     for (int w = 0; w < started; w++) th[w].join();
 }
 
+// Pinned slots of the process: a call takes what is free and allocates the
+// rest, and gives them back; at most two per possible worker stay, for as
+// long as any lattice lives (mrlbm_create and mrlbm_destroy count them). A
+// fresh slab of 16 MiB costs 0.4 ms to allocate and as much again on its first
+// use, a slot by itself about 15 us, and a living lattice's next transfer
+// nothing (create, two transfers and destroy of a 96x72x80 lattice: 3.7 ms
+// with a slab per call, 2.3 ms; slots in pairs of 2 MiB, past what the runtime
+// cuts from its own blocks, 4.8 ms).
+struct SlotPool {
+    static constexpr size_t KEPT = 2 * MAX_WORKERS;
+    std::mutex mu;
+    char* kept[KEPT];
+    size_t n = 0;
+    int lattices = 0;
+    hipError_t take(char** p) {
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            if (n) {
+                *p = kept[--n];
+                return hipSuccess;
+            }
+        }
+        return hipHostMalloc((void**)p, SLOT_BYTES, hipHostMallocPortable);
+    }
+    void give(char* p) {
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            if (lattices > 0 && n < KEPT) {
+                kept[n++] = p;
+                return;
+            }
+        }
+        (void)hipHostFree(p);
+    }
+    void count(int d) {
+        size_t m = 0;
+        char* drop[KEPT];
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            lattices += d;
+            if (lattices == 0) {
+                for (m = 0; m < n; m++) drop[m] = kept[m];
+                n = 0;
+            }
+        }
+        for (size_t k = 0; k < m; k++) (void)hipHostFree(drop[k]);
+    }
+};
+SlotPool g_slots;
+
 // Pinned slots and their events for one call.
 struct Slots {
-    char* mem = nullptr;
+    char* mem[2 * MAX_WORKERS] = {};
     hipEvent_t ev[2 * MAX_WORKERS] = {};
     int n = 0;
     hipError_t open(int slots) {
-        hipError_t e = hipHostMalloc((void**)&mem, SLOT_BYTES * (size_t)slots, hipHostMallocDefault);
-        if (e != hipSuccess) {
-            mem = nullptr;
-            return e;
+        for (; n < slots; n++) {
+            hipError_t e = g_slots.take(&mem[n]);
+            if (e != hipSuccess) return e;
+            if ((e = hipEventCreateWithFlags(&ev[n], hipEventDisableTiming)) != hipSuccess) {
+                g_slots.give(mem[n]);
+                return e;
+            }
         }
-        for (; n < slots; n++)
-            if ((e = hipEventCreateWithFlags(&ev[n], hipEventDisableTiming)) != hipSuccess) return e;
         return hipSuccess;
     }
     ~Slots() {
-        for (int k = 0; k < n; k++) (void)hipEventDestroy(ev[k]);
-        if (mem) (void)hipHostFree(mem);
+        for (int k = 0; k < n; k++) {
+            (void)hipEventDestroy(ev[k]);
+            g_slots.give(mem[k]);
+        }
     }
-    char* at(int k) const { return mem + SLOT_BYTES * (size_t)k; }
+    char* at(int k) const { return mem[k]; }
 };
 
 // Moves `chunks` chunks through pinned slots, worker w taking w, w + W, ...
@@ -98,7 +152,7 @@ int pump(mrlbm_ctx* c, size_t chunks, Launch&& launch, Take&& take) {
     if (chunks == 0) return MRLBM_OK;
     const int W = workers_for(chunks);
     Slots slots;
-    hipError_t e = slots.open(chunks == 1 ? 1 : 2 * W);
+    hipError_t e = slots.open((size_t)(2 * W) < chunks ? 2 * W : (int)chunks);
     if (e != hipSuccess) return fail(MRLBM_ENOMEM, "pinned staging memory: %s", hipGetErrorString(e));
     std::atomic<int> err{(int)hipSuccess};
     auto worker = [&](int w) {
@@ -294,9 +348,16 @@ int bad_density(const mrlbm_ctx* c, size_t j) {
 
 namespace mrlbm {
 
-int read_moments_linear(mrlbm_ctx* c, double* out) {
+void count_lattices(int d) { g_slots.count(d); }
+
+namespace {
+
+// The first `planes` stored moments; widen(o, in, n, plane) files n FP32
+// values of one plane.
+template <typename Widen>
+int read_planes(mrlbm_ctx* c, int planes, double* out, Widen&& widen) {
     const Linear L = linear_of(c);
-    const Chunks ch{(uint64_t)L.groups * 10, SLOT_BYTES / sizeof(f32x4)};
+    const Chunks ch{(uint64_t)L.groups * planes, SLOT_BYTES / sizeof(f32x4)};
     return pump<true>(
         c, ch.count(),
         [&](size_t k, char* slot) {
@@ -308,10 +369,32 @@ int read_moments_linear(mrlbm_ctx* c, double* out) {
         },
         [&](size_t k, const char* slot) {
             const float* in = (const float*)slot;
-            double* o = out + 4 * ch.first(k);
-            const size_t n = 4 * (size_t)ch.size(k);
-            for (size_t j = 0; j < n; j++) o[j] = in[j];
+            uint64_t at = 4 * ch.first(k);
+            const uint64_t end = at + 4 * (uint64_t)ch.size(k);
+            while (at < end) {  // a chunk of a small lattice spans planes
+                const uint64_t plane = at / c->N, stop = (plane + 1) * c->N < end ? (plane + 1) * c->N : end;
+                widen(out + at, in, (size_t)(stop - at), (int)plane);
+                in += stop - at;
+                at = stop;
+            }
         });
+}
+
+}  // namespace
+
+int read_moments_linear(mrlbm_ctx* c, double* out) {
+    return read_planes(c, 10, out, [](double* o, const float* in, size_t n, int) {
+        for (size_t j = 0; j < n; j++) o[j] = in[j];
+    });
+}
+
+int read_macroscopic_linear(mrlbm_ctx* c, double rho0, double* out) {
+    return read_planes(c, 4, out, [rho0](double* o, const float* in, size_t n, int plane) {
+        if (plane == 0)
+            for (size_t j = 0; j < n; j++) o[j] = (double)in[j] + rho0;
+        else
+            for (size_t j = 0; j < n; j++) o[j] = (double)in[j] / 3.0;
+    });
 }
 
 int write_moments_linear(mrlbm_ctx* c, const double* in) {

@@ -127,9 +127,9 @@ class Lattice:
 
     def macroscopic(self, rho0=1.0):
         """rho, ux, uy, uz as (nx, ny, nz) arrays (unscaled)."""
-        m = self.moments()
-        f = lambda v: v.reshape(self.shape, order="F")
-        return f(m[0] + rho0), f(m[1] / 3), f(m[2] / 3), f(m[3] / 3)
+        out = np.empty(4 * self.n)
+        _lib.check(_lib.load().mrlbm_read_macroscopic(self._h, float(rho0), out.ctypes.data_as(_lib._dp)))
+        return tuple(v.reshape(self.shape, order="F") for v in out.reshape(4, self.n))
 
     def reduce(self):
         """(mean(rho - rho0), mean(rho |u|^2 / 2)) in FP64."""

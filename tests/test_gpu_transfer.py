@@ -145,3 +145,47 @@ def test_bad_density_changes_nothing():
         with pytest.raises(mrlbm.MrlbmError, match="non-positive density"):
             lat.init_taylor_green(4.0)
         assert np.array_equal(lat.moments(), before)
+
+
+@pytest.mark.parametrize("storage", STORES)
+@pytest.mark.parametrize("shape,kw", SHAPES)
+def test_macroscopic_equals_moments(shape, kw, storage):
+    print("case", shape, storage, flush=True)
+    with lattice(shape, kw, storage) as lat:
+        lat.init_taylor_green(0.05)
+        lat.step(3)
+        m = lat.moments()
+        for rho0 in (1.0, 0.7):
+            got = lat.macroscopic(rho0)
+            want = [m[0] + rho0, m[1] / 3, m[2] / 3, m[3] / 3]
+            for g, w in zip(got, want):
+                assert g.shape == shape and np.array_equal(g.reshape(-1, order="F"), w)
+
+
+def test_transfers_of_several_threads():
+    """Threads move different lattices at the same time through the process's
+    pinned slots; lattices come and go meanwhile."""
+    import threading
+    shapes = [(72, 64, 80), (40, 24, 56), (64, 64, 64), (16, 8, 24)]
+    errors = []
+
+    def work(i):
+        try:
+            rng = np.random.default_rng(i)
+            for r in range(4):
+                shape = shapes[(i + r) % len(shapes)]
+                n = int(np.prod(shape))
+                with mrlbm.Lattice(shape, q=19, tau=0.6) as lat:
+                    m = rng.normal(size=(10, n)).astype(np.float32).astype(np.float64)
+                    lat.write_moments(m)
+                    if not np.array_equal(lat.moments(), m):
+                        errors.append((i, r, shape))
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    th = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not errors
