@@ -277,13 +277,44 @@ __device__ __forceinline__ void tile_fetch(const StepArgs& a, const float* gin, 
     });
 }
 
+// Arguments of a tile update from the boundary solve on.
+struct LateArgs {
+    const StepArgs& a;
+    float* gout;
+    uint32_t step;
+};
+
+// Those of a kernel whose first argument is its StepArgs. RELOAD: read from
+// the kernel's arguments again, through an address that the compiler takes
+// for new, so that they occupy no scalar registers until then. The D3Q27
+// kernel of both bodies needs that in the 16-bit formats: scalar registers
+// that did not fit took a vector register, and two ghost chunks were spilled,
+// each spill waiting for its load before the reconstruction could begin.
+// With the known masks in scalar registers too (KNOWN_SCALAR below), per
+// step, walls and two spheres: FP16 32^3 7.75 -> 7.04 us, 96x72x80
+// 17.7 -> 16.7, 200x72x104 32.4 -> 30.7, 256x256x128 153.6 -> 146.8,
+// 512x256x256 587 -> 577; BF16 (one chunk still spilled) 200x72x104
+// 32.4 -> 31.0, 512x256x256 589 -> 583. Elsewhere nothing is spilled and the
+// second read only costs (FP32 D3Q19 0.5-2 %).
+template <bool RELOAD>
+__device__ __forceinline__ LateArgs late_args(const StepArgs& first) {
+    if constexpr (RELOAD) {
+        auto p = (const __attribute__((address_space(4))) StepArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(p));
+        const StepArgs& a = *(const StepArgs*)p;
+        return {a, a.gout, a.step};
+    }
+    return {first, first.gout, first.step};
+}
+
 // One time step of one tile from its fetched inputs (the body of
 // k_step_tile and of the batched kernel). The whole workgroup calls it
 // with the same tile. `ahead` is called once the inputs are consumed
 // (before the first barrier): it issues the next tile's fetch.
-template <int Q, int BX, int BY, int BZ, bool HAS_BC, int S, typename Lds, typename Ahead>
-__device__ __forceinline__ void tile_update(const StepArgs& a, float* gout, uint32_t step, int tile, Lds& L,
-                                            const TileIn<Q, BX, BY, BZ, S>& in, Ahead&& ahead) {
+// `late` gives the arguments that the part after the streaming reads.
+template <int Q, int BX, int BY, int BZ, bool HAS_BC, int S, typename Lds, typename Ahead, typename Late>
+__device__ __forceinline__ void tile_update(const StepArgs& a, int tile, Lds& L,
+                                            const TileIn<Q, BX, BY, BZ, S>& in, Ahead&& ahead, Late&& late) {
     constexpr int T = BX * BY * BZ;
     constexpr int NW = T / 64;
     using G = HaloGeom<BX, BY, BZ>;
@@ -322,7 +353,12 @@ __device__ __forceinline__ void tile_update(const StepArgs& a, float* gout, uint
     const bool bcn = HAS_BC && cls != 0u && cls != 255u;
     const auto rec = gptr(a.bc) + (size_t)cls * BC_STRIDE;
     constexpr bool TWO_AHEAD = Q == 19;
-    uint32_t known = ~0u, uc0 = 0, uc1 = 0;
+    // 16-bit D3Q27 keeps the known-population masks of a wave's one or two
+    // classes in scalar registers until the solve (a vector register less
+    // while the populations are formed: FP16's kernel of both bodies spills
+    // nothing, see late_args)
+    constexpr bool KNOWN_SCALAR = Q == 27 && S != 0;
+    uint32_t known = ~0u, known0 = 0, known1 = 0, uc0 = 0, uc1 = 0;
     bool many = false;
     RowRecord rr{}, rr1{};
     auto row_record = [&](uint32_t uc, RowRecord& r) {
@@ -332,7 +368,7 @@ __device__ __forceinline__ void tile_update(const StepArgs& a, float* gout, uint
     const uint64_t bcw = HAS_BC ? __builtin_amdgcn_ballot_w64(bcn) : 0;
     if constexpr (HAS_BC) {
         if (bcw != 0) {  // uniform: waves without boundary nodes skip
-            if (bcn) known = __float_as_uint(rec[0]);
+            if (!KNOWN_SCALAR && bcn) known = __float_as_uint(rec[0]);
             uc0 = uc1 = (uint32_t)__builtin_amdgcn_readlane((int)cls, __builtin_ctzll(bcw));
             uint64_t rest = bcw & ~__builtin_amdgcn_ballot_w64(cls == uc0);
             if (rest != 0) {
@@ -343,6 +379,10 @@ __device__ __forceinline__ void tile_update(const StepArgs& a, float* gout, uint
             if (!many) {
                 row_record(uc0, rr);
                 if (TWO_AHEAD && uc1 != uc0) row_record(uc1, rr1);
+                if constexpr (KNOWN_SCALAR) {
+                    known0 = __float_as_uint(gptr(a.bc)[(size_t)uc0 * BC_STRIDE]);
+                    known1 = __float_as_uint(gptr(a.bc)[(size_t)uc1 * BC_STRIDE]);
+                }
             }
         }
     }
@@ -433,20 +473,23 @@ __device__ __forceinline__ void tile_update(const StepArgs& a, float* gout, uint
         });
     });
 
+    const LateArgs la = late();
+    const StepArgs& al = la.a;
     Node m;
     if constexpr (HAS_BC) {
         // boundary nodes: one pass of moment sums shared with the bulk nodes
         // of the wave, over their known populations only (the others zeroed)
+        if (KNOWN_SCALAR && bcn) known = many ? __float_as_uint(rec[0]) : (cls == uc0 ? known0 : known1);
         if (bcw != 0) known_only<Q>(known, g);
         Sums sums;
         moment_sums<Q>(g, sums);
-        bulk_from_sums(sums, a.rho0, m, SU, SM);
+        bulk_from_sums(sums, al.rho0, m, SU, SM);
         if (bcw != 0) {
             if (!many) {
 #pragma unroll 1
                 for (uint32_t uc = uc0;; uc = uc1) {
                     Node b;
-                    bc_from_sums(rr, sums, a.rho0, b);
+                    bc_from_sums(rr, sums, al.rho0, b);
                     scale_moments(b, SU, SM);
                     // every lane computes it (the broadcasts need the whole
                     // wave): keep the arithmetic out of the branch below
@@ -461,33 +504,33 @@ __device__ __forceinline__ void tile_update(const StepArgs& a, float* gout, uint
                         row_record(uc1, rr);
                 }
             } else if (bcn) {
-                bc_from_sums(PointerRecord<decltype(rec)>{rec}, sums, a.rho0, m);
+                bc_from_sums(PointerRecord<decltype(rec)>{rec}, sums, al.rho0, m);
                 scale_moments(m, SU, SM);
             }
         }
     } else {
-        bulk_moments<Q>(g, a.rho0, m, SU, SM);
+        bulk_moments<Q>(g, al.rho0, m, SU, SM);
     }
-    collide(m, a.R);
+    collide(m, al.R);
     typename Codec<S>::T q[10];
     // global node index x + nx (y + ny z), mod 2^32: tz is uniform in a wave
     // (waves cover whole x rows, BX * BY is a multiple of 64), so only
     // tx + nx ty is per-lane arithmetic (24-bit multiply: nx < 2^24)
     static_assert((BX * BY) % 64 == 0, "a wave spans whole xy-plane rows");
-    const uint32_t nxu = (uint32_t)a.nx, nxy = nxu * (uint32_t)a.ny;
+    const uint32_t nxu = (uint32_t)al.nx, nxy = nxu * (uint32_t)al.ny;
     const uint32_t zw = (uint32_t)(bz * BZ) + (uint32_t)__builtin_amdgcn_readfirstlane(tz);
     const uint32_t node_id = ((uint32_t)(bx * BX) + nxu * (uint32_t)(by * BY) + nxy * zw) + ((uint32_t)tx + __umul24(nxu, (uint32_t)ty));
     Recon rt;
     if constexpr (F16) {
         uint32_t pk[5];
-        quantize<S>(m, a, step, node_id, q, pk);
+        quantize<S>(m, al, la.step, node_id, q, pk);
         float re0;
-        recon_terms_f16<Q, true>(pk, a.rho0, m.drho, m.rho, re0, rt);
+        recon_terms_f16<Q, true>(pk, al.rho0, m.drho, m.rho, re0, rt);
     } else {
-        quantize<S>(m, a, step, node_id, q);
+        quantize<S>(m, al, la.step, node_id, q);
         recon_terms<Q>(m, recon_re0<Q>(m), rt);
     }
-    if (!solid) store_tile_node<BX, BY, BZ, S>(a, tile, t, q);
+    if (!solid) store_tile_node<BX, BY, BZ, S>(al, tile, t, q);
 
     // populations leaving the tile (popSave.inc): every node stages its
     // reconstruction terms in LDS, then whole waves evaluate and write the
@@ -506,7 +549,7 @@ __device__ __forceinline__ void tile_update(const StepArgs& a, float* gout, uint
         static_for<(NOUT + NW - 1) / NW>([&](auto RR) {
             constexpr int K = W + NW * decltype(RR)::value;
             if constexpr (K < NOUT)
-                halo_store<Q, BX, BY, BZ, HAS_BC, K>(a, gout, lane, tile, bx, by, bz, s, s_cls);
+                halo_store<Q, BX, BY, BZ, HAS_BC, K>(al, la.gout, lane, tile, bx, by, bz, s, s_cls);
         });
     });
 }
@@ -552,7 +595,7 @@ void k_step_tile(StepArgs a, const uint32_t* __restrict__ list) {
                           : (int)xcd_grouped(blockIdx.x, a.group_end);
     TileIn<Q, BX, BY, BZ, S> in;
     tile_fetch<Q, BX, BY, BZ, HAS_BC, S>(a, a.gin, tile, in);
-    tile_update<Q, BX, BY, BZ, HAS_BC, S>(a, a.gout, a.step, tile, L, in, []() {});
+    tile_update<Q, BX, BY, BZ, HAS_BC, S>(a, tile, L, in, []() {}, [&]() { return late_args<false>(a); });
 }
 
 // Batched step: each block takes a contiguous range of work items (the
@@ -588,12 +631,12 @@ void k_step_batch(const InstArgs* __restrict__ tab,
         int ninst = inst, ntile = tile;
         if (item + 1 < end) item_of(item + 1, ninst, ntile);
         In nx;
-        tile_update<Q, BX, BY, BZ, HAS_BC, S>(ia.a, ia.g[1 - p], ia.step0 + (uint32_t)k, tile, L, in, [&]() {
+        tile_update<Q, BX, BY, BZ, HAS_BC, S>(ia.a, tile, L, in, [&]() {
             if (item + 1 < end) {
                 const InstArgs& nia = tab[ninst];
                 tile_fetch<Q, BX, BY, BZ, HAS_BC, S>(nia.a, nia.g[(nia.cur0 + k) & 1], ntile, nx);
             }
-        });
+        }, [&]() { return LateArgs{ia.a, ia.g[1 - p], ia.step0 + (uint32_t)k}; });
         __syncthreads();  // LDS is reused by the next item
         in = nx;
         inst = ninst;
@@ -615,7 +658,9 @@ void k_step_batch1(const InstArgs* __restrict__ tab, const uint32_t* __restrict_
     const int p = (ia.cur0 + k) & 1;
     TileIn<Q, BX, BY, BZ, S> in;
     tile_fetch<Q, BX, BY, BZ, HAS_BC, S>(ia.a, ia.g[p], tile, in);
-    tile_update<Q, BX, BY, BZ, HAS_BC, S>(ia.a, ia.g[1 - p], ia.step0 + (uint32_t)k, tile, L, in, []() {});
+    tile_update<Q, BX, BY, BZ, HAS_BC, S>(ia.a, tile, L, in, []() {}, [&]() {
+            return LateArgs{ia.a, ia.g[1 - p], ia.step0 + (uint32_t)k};
+        });
 }
 
 // Both bodies in one launch, where they run at the same occupancy (the same
@@ -634,15 +679,16 @@ template <int Q, int BX, int BY, int BZ, int S>
 __global__ __launch_bounds__(BX* BY* BZ) __attribute__((amdgpu_waves_per_eu(step_body_waves<Q, BX, BY, BZ, true, S>())))
 void k_step_tile_mixed(StepArgs a, const uint32_t* __restrict__ list, int nbulk) {
     __shared__ TileLds<Q, BX, BY, BZ, true> L;
+    constexpr bool RELOAD = Q == 27 && S != 0;
     const int tile = (int)__builtin_amdgcn_readfirstlane(list[blockIdx.x]);
     if ((int)blockIdx.x < nbulk) {
         TileIn<Q, BX, BY, BZ, S> in;
         tile_fetch<Q, BX, BY, BZ, false, S>(a, a.gin, tile, in);
-        tile_update<Q, BX, BY, BZ, false, S>(a, a.gout, a.step, tile, L, in, []() {});
+        tile_update<Q, BX, BY, BZ, false, S>(a, tile, L, in, []() {}, [&]() { return late_args<RELOAD>(a); });
     } else {
         TileIn<Q, BX, BY, BZ, S> in;
         tile_fetch<Q, BX, BY, BZ, true, S>(a, a.gin, tile, in);
-        tile_update<Q, BX, BY, BZ, true, S>(a, a.gout, a.step, tile, L, in, []() {});
+        tile_update<Q, BX, BY, BZ, true, S>(a, tile, L, in, []() {}, [&]() { return late_args<RELOAD>(a); });
     }
 }
 
@@ -657,11 +703,15 @@ void k_step_batch1_mixed(const InstArgs* __restrict__ tab, const uint32_t* __res
     if ((int)blockIdx.x < nbulk) {
         TileIn<Q, BX, BY, BZ, S> in;
         tile_fetch<Q, BX, BY, BZ, false, S>(ia.a, ia.g[p], tile, in);
-        tile_update<Q, BX, BY, BZ, false, S>(ia.a, ia.g[1 - p], ia.step0 + (uint32_t)k, tile, L, in, []() {});
+        tile_update<Q, BX, BY, BZ, false, S>(ia.a, tile, L, in, []() {}, [&]() {
+            return LateArgs{ia.a, ia.g[1 - p], ia.step0 + (uint32_t)k};
+        });
     } else {
         TileIn<Q, BX, BY, BZ, S> in;
         tile_fetch<Q, BX, BY, BZ, true, S>(ia.a, ia.g[p], tile, in);
-        tile_update<Q, BX, BY, BZ, true, S>(ia.a, ia.g[1 - p], ia.step0 + (uint32_t)k, tile, L, in, []() {});
+        tile_update<Q, BX, BY, BZ, true, S>(ia.a, tile, L, in, []() {}, [&]() {
+            return LateArgs{ia.a, ia.g[1 - p], ia.step0 + (uint32_t)k};
+        });
     }
 }
 
