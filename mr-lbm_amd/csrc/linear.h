@@ -171,11 +171,13 @@ __device__ __forceinline__ void block_sum(double (&v)[K]) {
             for (int j = 1; j < RED_THREADS / 64; j++) v[k] += w[j][k];
 }
 
-// x / 3 to within rounding: a product with 1/3 and one correction (an FP64
-// division takes several times as many instructions).
-__device__ __forceinline__ double third(double x) {
+// x / 3 for x of a 32-bit value: a product with 1/3 and one correction (an FP64
+// division takes several times as many instructions). For an infinite x the
+// correction would be inf - inf; the product is the quotient then.
+__host__ __device__ __forceinline__ double third(double x) {
     const double q = x * (1.0 / 3.0);
-    return __builtin_fma(__builtin_fma(-3.0, q, x), 1.0 / 3.0, q);
+    const double r = __builtin_fma(__builtin_fma(-3.0, q, x), 1.0 / 3.0, q);
+    return __builtin_isinf(x) ? q : r;
 }
 
 // Fold n partial records of K sums (record b at partial[K b]) in a fixed

@@ -80,3 +80,29 @@ def test_non_finite_nodes_are_counted(storage):
         m[5, 77] = np.inf  # a second moment does not count
         lat.write_moments(m)
         assert lat.reduce_checked()[2] == 5
+
+
+@pytest.mark.parametrize("storage", [mrlbm.STORE_FP32, mrlbm.STORE_FP16, mrlbm.STORE_BF16])
+def test_infinite_velocities_stay_infinite_in_the_mean_flow(storage):
+    with mrlbm.Lattice((40, 16, 24), q=19, tau=0.6, storage=storage) as lat:
+        lat.init_uniform(u=(0.03, 0.0, 0.0))
+        m = lat.moments()
+        at = {(1, 0): np.inf, (2, 7): -np.inf, (3, 8191): np.inf, (1, lat.n - 1): -np.inf, (2, 500): np.nan}
+        for (row, node), v in at.items():
+            m[row, node] = v
+        lat.write_moments(m)
+        held = lat.moments()
+        for key, v in at.items():
+            assert np.array_equal(held[key], v, equal_nan=True)
+        for _ in range(2):
+            lat.mean_flow_accumulate()
+        u = np.stack([f.reshape(-1, order="F") for f in lat.mean_flow()[0][1:]])
+        assert np.array_equal(u, held[1:4] / 3.0, equal_nan=True)
+        # against a finite mean an infinite velocity has infinite energy
+        lat.mean_flow_reset()
+        lat.init_uniform(u=(0.03, 0.0, 0.0))
+        lat.mean_flow_accumulate()
+        m = lat.moments()
+        m[1, 77] = np.inf
+        lat.write_moments(m)
+        assert lat.turbulent_ke() == np.inf
