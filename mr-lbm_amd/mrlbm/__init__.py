@@ -126,10 +126,18 @@ class Lattice:
         _lib.check(_lib.load().mrlbm_write_moments(self._h, m.ctypes.data_as(_lib._dp)))
 
     def macroscopic(self, rho0=1.0):
-        """rho, ux, uy, uz as (nx, ny, nz) arrays (unscaled)."""
+        """rho, ux, uy, uz as (nx, ny, nz) arrays (unscaled). rho0 is what the
+        stored rho - RHO_0 is added to: a number, or an array in x-fastest
+        order (anything that adds to N values)."""
+        number = isinstance(rho0, (int, float))
         out = np.empty(4 * self.n)
-        _lib.check(_lib.load().mrlbm_read_macroscopic(self._h, float(rho0), out.ctypes.data_as(_lib._dp)))
-        return tuple(v.reshape(self.shape, order="F") for v in out.reshape(4, self.n))
+        # x + -0.0 is x, of either sign of zero
+        _lib.check(_lib.load().mrlbm_read_macroscopic(self._h, float(rho0) if number else -0.0,
+                                                      out.ctypes.data_as(_lib._dp)))
+        rho, *u = out.reshape(4, self.n)
+        if not number:
+            rho = rho + rho0
+        return tuple(v.reshape(self.shape, order="F") for v in (rho, *u))
 
     def reduce(self):
         """(mean(rho - rho0), mean(rho |u|^2 / 2)) in FP64."""

@@ -189,3 +189,28 @@ def test_transfers_of_several_threads():
     for t in th:
         t.join()
     assert not errors
+
+
+def test_macroscopic_adds_any_density():
+    """rho0 as numpy takes it in a sum: arrays, lists and scalar types; what a
+    sum refuses is refused."""
+    shape = (24, 16, 8)
+    n = int(np.prod(shape))
+    with lattice(shape, {}) as lat:
+        lat.init_taylor_green(0.05)
+        lat.step(3)
+        m = lat.moments()
+        rng = np.random.default_rng(1)
+        for rho0 in (rng.uniform(0.9, 1.1, n), rng.uniform(0.9, 1.1, n).astype(np.float32), np.array([0.8]), [0.5],
+                     np.arange(n), np.float32(0.7), np.array(0.3), 1, True, -0.0, np.float64(1.0), 1.0 + 2.0j):
+            rho, *u = lat.macroscopic(rho0)
+            want = m[0] + rho0
+            assert rho.shape == shape and rho.dtype == want.dtype
+            assert np.array_equal(rho.reshape(-1, order="F"), want)
+            for a in range(3):
+                assert np.array_equal(u[a].reshape(-1, order="F"), m[1 + a] / 3)
+        for rho0 in (None, "1.0", np.ones(n - 1)):
+            with pytest.raises((TypeError, ValueError)):
+                m[0] + rho0
+            with pytest.raises((TypeError, ValueError)):
+                lat.macroscopic(rho0)
