@@ -148,6 +148,8 @@ int mrlbm_read_moments(mrlbm_ctx* ctx, double* out10n);
  * rho-RHO_0 plus rho0, and the stored 3u over 3 (the fields that saveMacr
  * writes, src/saveData.cu:7-260), without the second moments. */
 int mrlbm_read_macroscopic(mrlbm_ctx* ctx, double rho0, double* out4n);
+/* The same into four arrays of N values, as mrlbm_init_fields takes them. */
+int mrlbm_read_fields(mrlbm_ctx* ctx, double rho0, double* rho, double* ux, double* uy, double* uz);
 
 /* Overwrite the stored moments (same format) and rebuild both ghost sets
  * from them, as gpuInitialization_pop does. */

@@ -393,7 +393,14 @@ int mrlbm_read_moments(mrlbm_ctx* c, double* out) {
 
 int mrlbm_read_macroscopic(mrlbm_ctx* c, double rho0, double* out) {
     if (!c || !out) return fail(MRLBM_EINVAL, "null argument");
-    return read_macroscopic_linear(c, rho0, out);
+    double* const plane[4] = {out, out + c->N, out + 2 * c->N, out + 3 * c->N};
+    return read_macroscopic_linear(c, rho0, plane);
+}
+
+int mrlbm_read_fields(mrlbm_ctx* c, double rho0, double* rho, double* ux, double* uy, double* uz) {
+    if (!c || !rho || !ux || !uy || !uz) return fail(MRLBM_EINVAL, "null argument");
+    double* const plane[4] = {rho, ux, uy, uz};
+    return read_macroscopic_linear(c, rho0, plane);
 }
 
 int mrlbm_write_moments(mrlbm_ctx* c, const double* in) {

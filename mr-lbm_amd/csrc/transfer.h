@@ -14,8 +14,8 @@ void count_lattices(int d);
 
 // Stored moments decoded into out[k * N + x + NX (y + NY z)].
 int read_moments_linear(mrlbm_ctx* c, double* out);
-// rho0 + (rho - RHO_0), ux, uy, uz: four such planes.
-int read_macroscopic_linear(mrlbm_ctx* c, double rho0, double* out);
+// rho0 + (rho - RHO_0), ux, uy, uz: four such planes, each by itself.
+int read_macroscopic_linear(mrlbm_ctx* c, double rho0, double* const out[4]);
 // Stored moments from the same layout.
 int write_moments_linear(mrlbm_ctx* c, const double* in);
 // Stored moments from density and velocity fields; refuses a non-positive

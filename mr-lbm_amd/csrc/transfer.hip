@@ -352,10 +352,10 @@ void count_lattices(int d) { g_slots.count(d); }
 
 namespace {
 
-// The first `planes` stored moments; widen(o, in, n, plane) files n FP32
-// values of one plane.
+// The first `planes` stored moments, plane k into out[k]; widen(o, in, n,
+// plane) files n FP32 values of one plane.
 template <typename Widen>
-int read_planes(mrlbm_ctx* c, int planes, double* out, Widen&& widen) {
+int read_planes(mrlbm_ctx* c, int planes, double* const* out, Widen&& widen) {
     const Linear L = linear_of(c);
     const Chunks ch{(uint64_t)L.groups * planes, SLOT_BYTES / sizeof(f32x4)};
     return pump<true>(
@@ -373,7 +373,7 @@ int read_planes(mrlbm_ctx* c, int planes, double* out, Widen&& widen) {
             const uint64_t end = at + 4 * (uint64_t)ch.size(k);
             while (at < end) {  // a chunk of a small lattice spans planes
                 const uint64_t plane = at / c->N, stop = (plane + 1) * c->N < end ? (plane + 1) * c->N : end;
-                widen(out + at, in, (size_t)(stop - at), (int)plane);
+                widen(out[plane] + (at - plane * c->N), in, (size_t)(stop - at), (int)plane);
                 in += stop - at;
                 at = stop;
             }
@@ -383,12 +383,14 @@ int read_planes(mrlbm_ctx* c, int planes, double* out, Widen&& widen) {
 }  // namespace
 
 int read_moments_linear(mrlbm_ctx* c, double* out) {
-    return read_planes(c, 10, out, [](double* o, const float* in, size_t n, int) {
+    double* plane[10];
+    for (int k = 0; k < 10; k++) plane[k] = out + (size_t)k * c->N;
+    return read_planes(c, 10, plane, [](double* o, const float* in, size_t n, int) {
         for (size_t j = 0; j < n; j++) o[j] = in[j];
     });
 }
 
-int read_macroscopic_linear(mrlbm_ctx* c, double rho0, double* out) {
+int read_macroscopic_linear(mrlbm_ctx* c, double rho0, double* const out[4]) {
     return read_planes(c, 4, out, [rho0](double* o, const float* in, size_t n, int plane) {
         if (plane == 0)
             for (size_t j = 0; j < n; j++) o[j] = (double)in[j] + rho0;

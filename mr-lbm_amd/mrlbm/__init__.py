@@ -130,11 +130,10 @@ class Lattice:
         stored rho - RHO_0 is added to: a number, or an array in x-fastest
         order (anything that adds to N values)."""
         number = isinstance(rho0, (int, float))
-        out = np.empty(4 * self.n)
+        rho, *u = [np.empty(self.n) for _ in range(4)]
         # x + -0.0 is x, of either sign of zero
-        _lib.check(_lib.load().mrlbm_read_macroscopic(self._h, float(rho0) if number else -0.0,
-                                                      out.ctypes.data_as(_lib._dp)))
-        rho, *u = out.reshape(4, self.n)
+        _lib.check(_lib.load().mrlbm_read_fields(self._h, float(rho0) if number else -0.0,
+                                                 *[v.ctypes.data_as(_lib._dp) for v in (rho, *u)]))
         if not number:
             rho = rho + rho0
         return tuple(v.reshape(self.shape, order="F") for v in (rho, *u))

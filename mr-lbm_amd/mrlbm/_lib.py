@@ -96,6 +96,7 @@ _SIGS = {
     "mrlbm_synchronize": [_vp],
     "mrlbm_read_moments": [_vp, _dp],
     "mrlbm_read_macroscopic": [_vp, ctypes.c_double, _dp],
+    "mrlbm_read_fields": [_vp, ctypes.c_double, _dp, _dp, _dp, _dp],
     "mrlbm_write_moments": [_vp, _dp],
     "mrlbm_reduce": [_vp, _dp, _dp],
     "mrlbm_reduce_checked": [_vp, _dp, _dp, ctypes.POINTER(ctypes.c_int64)],

@@ -214,3 +214,18 @@ def test_macroscopic_adds_any_density():
                 m[0] + rho0
             with pytest.raises((TypeError, ValueError)):
                 lat.macroscopic(rho0)
+
+
+def test_macroscopic_fields_own_their_memory():
+    """A field that is kept does not keep the others; the C entry with one
+    buffer gives the same values."""
+    with lattice((40, 24, 56), {}) as lat:
+        lat.init_taylor_green(0.05)
+        lat.step(3)
+        got = lat.macroscopic(0.9)
+        for f in got:
+            assert f.base is not None and f.base.nbytes == 8 * lat.n
+        one = np.empty((4, lat.n))
+        mrlbm._lib.check(mrlbm._lib.load().mrlbm_read_macroscopic(lat._h, 0.9, one.ctypes.data_as(mrlbm._lib._dp)))
+        for f, w in zip(got, one):
+            assert np.array_equal(f.reshape(-1, order="F"), w)
