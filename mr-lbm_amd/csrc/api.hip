@@ -412,6 +412,7 @@ int mrlbm_write_moments(mrlbm_ctx* c, const double* in) {
 int mrlbm_reduce_checked(mrlbm_ctx* c, double* mass, double* ke, int64_t* nonfinite) {
     if (!c || !mass || !ke || !nonfinite) return fail(MRLBM_EINVAL, "null argument");
     HIPCHK(hipSetDevice(c->p.device));
+    std::lock_guard<std::mutex> lock(c->small_mu);
     if (int rc = small_buffer(c)) return rc;
     double* const h = (double*)c->h_small;
     HIPCHK(launch_reduce(c->p.storage, c->d_mom, c->ntiles, c->T, (float)c->p.rho0, c->mrscale[0], c->mrscale[1],
@@ -442,6 +443,7 @@ int mrlbm_velocity_residual(mrlbm_ctx* c, double* residual) {
         c->device_bytes += (double)bytes;
         HIPCHK(hipMemsetAsync(c->d_uprev, 0, bytes, c->stream));
     }
+    std::lock_guard<std::mutex> lock(c->small_mu);
     if (int rc = small_buffer(c)) return rc;
     double* const h = (double*)c->h_small;
     HIPCHK(launch_residual(c->p.storage, c->d_mom, c->d_uprev, c->ntiles, c->T, c->mrscale[1], c->d_partial, h,

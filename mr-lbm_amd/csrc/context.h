@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -44,6 +45,7 @@ struct mrlbm_ctx {
     double bc_vel[4][3] = {};
     double* d_partial = nullptr;  // partial sums: 1024 records of at most ten values
     char* h_small = nullptr;      // pinned: results of sums, sample points and values (SMALL_BYTES, on first use)
+    std::mutex small_mu;          // held by a call that uses h_small, until it has read its results
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     double device_bytes = 0;
     mrlbm_batch* batch = nullptr;  // batch this lattice is stepped in (its stream is then the batch's)
@@ -144,6 +146,9 @@ hipStream_t batch_stream(const mrlbm_batch* b);
 
 // The context's small pinned buffer, which kernels read and write in place: a
 // result is on the host when the stream is idle, without a copy of its own.
+// The caller holds small_mu: threads that sample one lattice at the same time
+// (safe with a buffer per call) would read each other's points, and points
+// overwritten by another call's values are indices out of range.
 constexpr size_t SMALL_BYTES = 64 * 1024;
 int small_buffer(mrlbm_ctx* c);
 

@@ -147,6 +147,7 @@ int mrlbm_sample(mrlbm_ctx* c, int n, const int32_t* xyz, double* out) {
     // and two frees (16 points: 63 -> 18 us per call).
     constexpr int IN_PLACE = (int)(SMALL_BYTES / (10 * sizeof(double) + 3 * sizeof(int)));
     if (n <= IN_PLACE) {
+        std::lock_guard<std::mutex> lock(c->small_mu);
         if (int rc = small_buffer(c)) return rc;
         double* const h_out = (double*)c->h_small;
         int* const h_xyz = (int*)(h_out + 10 * (size_t)n);
@@ -173,6 +174,7 @@ int mrlbm_moment_means(mrlbm_ctx* c, double out[10]) {
     if (!c || !out) return fail(MRLBM_EINVAL, "null argument");
     if (!c->initialised) return fail(MRLBM_ESTATE, "lattice not initialised");
     HIPCHK(hipSetDevice(c->p.device));
+    std::lock_guard<std::mutex> lock(c->small_mu);
     if (int rc = small_buffer(c)) return rc;
     const BlockGroups g = block_groups((size_t)c->ntiles, c->T);
     const int nb = red_blocks(g.n);
@@ -218,6 +220,7 @@ int mrlbm_turbulent_ke(mrlbm_ctx* c, double* tke) {
     if (!c || !tke) return fail(MRLBM_EINVAL, "null argument");
     if (!c->d_mean || c->mean_count == 0) return fail(MRLBM_ESTATE, "no mean-flow samples accumulated");
     HIPCHK(hipSetDevice(c->p.device));
+    std::lock_guard<std::mutex> lock(c->small_mu);
     if (int rc = small_buffer(c)) return rc;
     const Patches P = patches_of(c);
     const int nb = red_blocks(P.n);

@@ -106,3 +106,45 @@ def test_infinite_velocities_stay_infinite_in_the_mean_flow(storage):
         m[1, 77] = np.inf
         lat.write_moments(m)
         assert lat.turbulent_ke() == np.inf
+
+
+def test_threads_read_one_lattice():
+    """Sampling and sums of one lattice from several threads at a time share
+    its result buffer: each call gets its own values."""
+    import threading
+    shape = (32, 24, 16)
+    errors = []
+    with mrlbm.Lattice(shape, q=19, tau=0.56) as lat:
+        lat.init_taylor_green(0.05)
+        lat.step(5)
+        lat.mean_flow_accumulate()
+        lat.step(2)
+        m = lat.moments()
+        sums = {"reduce_checked": lat.reduce_checked(), "moment_means": lat.moment_means(),
+                "turbulent_ke": lat.turbulent_ke()}
+
+        def sample(n):
+            rng = np.random.default_rng(n)
+            for _ in range(150):
+                p = np.stack([rng.integers(0, s, n) for s in shape], axis=1)
+                if not np.array_equal(lat.sample(p), m[:, p[:, 0] + 32 * (p[:, 1] + 24 * p[:, 2])].T):
+                    errors.append(n)
+
+        def total(name):
+            for _ in range(150):
+                if not np.array_equal(getattr(lat, name)(), sums[name]):
+                    errors.append(name)
+
+        def run(f, arg):
+            try:
+                f(arg)
+            except Exception as e:  # noqa: BLE001
+                errors.append(e)
+
+        th = [threading.Thread(target=run, args=(sample, n)) for n in (1, 16, 300, 712)]
+        th += [threading.Thread(target=run, args=(total, name)) for name in sums]
+        for t in th:
+            t.start()
+        for t in th:
+            t.join()
+    assert not errors
