@@ -433,6 +433,9 @@ int mrlbm_velocity_residual(mrlbm_ctx* c, double* residual) {
     if (!c || !residual) return fail(MRLBM_EINVAL, "null argument");
     if (!c->initialised) return fail(MRLBM_ESTATE, "lattice not initialised");
     HIPCHK(hipSetDevice(c->p.device));
+    std::lock_guard<std::mutex> lock(c->small_mu);
+    // before the reference: a call that fails here leaves the next one the first
+    if (int rc = small_buffer(c)) return rc;
     const bool first = c->d_uprev == nullptr;
     if (first) {
         const size_t bytes = sizeof(float) * 3 * c->N;
@@ -443,8 +446,6 @@ int mrlbm_velocity_residual(mrlbm_ctx* c, double* residual) {
         c->device_bytes += (double)bytes;
         HIPCHK(hipMemsetAsync(c->d_uprev, 0, bytes, c->stream));
     }
-    std::lock_guard<std::mutex> lock(c->small_mu);
-    if (int rc = small_buffer(c)) return rc;
     double* const h = (double*)c->h_small;
     HIPCHK(launch_residual(c->p.storage, c->d_mom, c->d_uprev, c->ntiles, c->T, c->mrscale[1], c->d_partial, h,
                            c->stream));
