@@ -37,34 +37,42 @@ constexpr int THREADS = 256;
 // one overlaps the transfer of the other. 1 MiB is the smallest size that
 // still moves at the PCIe rate (50 GB/s back to back; 256 KiB: 36 GB/s).
 constexpr size_t SLOT_BYTES = 1u << 20;
-// One core widens 22 GB/s into fresh memory, four 50 GB/s, eight 76 GB/s
-// (measured; PCIe delivers 108 GB/s of widened values): more than eight add
-// nothing. A worker is worth its thread (60 us to start and join) from about
-// three slots on.
-constexpr int MAX_WORKERS = 8;
-constexpr size_t CHUNKS_PER_WORKER = 3;
 
-int workers_for(size_t chunks) {
-    const unsigned hw = std::thread::hardware_concurrency();
-    size_t w = chunks / CHUNKS_PER_WORKER;
-    if (w > MAX_WORKERS) w = MAX_WORKERS;
-    if (hw && w > hw) w = hw;
-    return w < 1 ? 1 : (int)w;
-}
-
-// f(0) .. f(n - 1), each on a thread of its own (the last on the caller's);
-// where no thread can be started the caller runs the rest.
-template <typename F>
-void run_workers(int n, F&& f) {
-    std::thread th[MAX_WORKERS];
-    int started = 0;
-    try {
-        for (; started < n - 1; started++) th[started] = std::thread([&f, started] { f(started); });
-    } catch (const std::system_error&) {
-    } catch (const std::bad_alloc&) {
-    }
-    for (int w = started; w < n; w++) f(w);
-    for (int w = 0; w < started; w++) th[w].join();
+// Runs step() until it returns false, on the caller's thread and on helpers
+// that join it as processors are free for them: transfer_workers says how
+// many, asked after the caller's second step and after every eighth from there
+// on (left() is the number of chunks to go). Before a helper starts, grow()
+// provides for it on the caller's thread; the helper calls enter() first.
+// Either may decline.
+template <typename Left, typename Grow, typename Enter, typename Step>
+void run_workers(Left&& left, Grow&& grow, Enter&& enter, Step&& step) {
+    std::thread th[MAX_WORKERS - 1];
+    int have = 1;
+    auto helper = [&] {
+        if (enter())
+            while (step()) {
+            }
+    };
+    auto join_in = [&] {
+        const size_t l = left();
+        if (l < (have + 1) * CHUNKS_PER_WORKER) return true;
+        const int want = transfer_workers(l, std::thread::hardware_concurrency(), running_threads(), have);
+        for (; have < want; have++) {
+            if (!grow()) return false;
+            try {
+                th[have - 1] = std::thread(helper);
+            } catch (const std::system_error&) {
+                return false;
+            } catch (const std::bad_alloc&) {
+                return false;
+            }
+        }
+        return true;
+    };
+    bool more = true;
+    for (size_t n = 1; step(); n++)
+        if (more && n % 8 == 2) more = join_in();
+    for (int w = 1; w < have; w++) th[w - 1].join();
 }
 
 // Pinned slots of the process: a call takes what is free and allocates the
@@ -122,15 +130,14 @@ struct Slots {
     char* mem[2 * MAX_WORKERS] = {};
     hipEvent_t ev[2 * MAX_WORKERS] = {};
     int n = 0;
-    hipError_t open(int slots) {
-        for (; n < slots; n++) {
-            hipError_t e = g_slots.take(&mem[n]);
-            if (e != hipSuccess) return e;
-            if ((e = hipEventCreateWithFlags(&ev[n], hipEventDisableTiming)) != hipSuccess) {
-                g_slots.give(mem[n]);
-                return e;
-            }
+    hipError_t add() {
+        hipError_t e = g_slots.take(&mem[n]);
+        if (e != hipSuccess) return e;
+        if ((e = hipEventCreateWithFlags(&ev[n], hipEventDisableTiming)) != hipSuccess) {
+            g_slots.give(mem[n]);
+            return e;
         }
+        n++;
         return hipSuccess;
     }
     ~Slots() {
@@ -139,56 +146,83 @@ struct Slots {
             g_slots.give(mem[k]);
         }
     }
-    char* at(int k) const { return mem[k]; }
 };
 
-// Moves `chunks` chunks through pinned slots, worker w taking w, w + W, ...
-// DOWN: launch(c, slot) makes the device fill the slot, take(c, slot) empties
-// it on the host; otherwise take fills it and launch makes the device read
-// it. Returns when every chunk has arrived and the stream is idle.
+// Moves `chunks` chunks through pinned slots. DOWN: launch(c, slot) makes the
+// device fill the slot, take(c, slot) empties it on the host; otherwise take
+// fills it and launch makes the device read it. A worker takes the next chunk
+// when it is free, so one that the scheduler holds up keeps back a single
+// chunk. Returns when every chunk has arrived and the stream is idle.
 template <bool DOWN, typename Launch, typename Take>
 int pump(mrlbm_ctx* c, size_t chunks, Launch&& launch, Take&& take) {
     HIPCHK(hipSetDevice(c->p.device));
     if (chunks == 0) return MRLBM_OK;
-    const int W = workers_for(chunks);
     Slots slots;
-    hipError_t e = slots.open((size_t)(2 * W) < chunks ? 2 * W : (int)chunks);
-    if (e != hipSuccess) return fail(MRLBM_ENOMEM, "pinned staging memory: %s", hipGetErrorString(e));
-    std::atomic<int> err{(int)hipSuccess};
-    auto worker = [&](int w) {
-        auto ok = [&](hipError_t r) {
-            if (r != hipSuccess) err = (int)r;
-            return r == hipSuccess;
-        };
-        if (!ok(hipSetDevice(c->p.device))) return;
-        auto send = [&](size_t k, int s) { return ok(launch(k, slots.at(s))) && ok(hipEventRecord(slots.ev[s], c->stream)); };
-        if constexpr (DOWN) {
-            size_t ahead = w;
-            for (int b = 0; b < 2 && ahead < chunks; b++, ahead += W)
-                if (!send(ahead, 2 * w + b)) return;
-            for (size_t k = w, b = 0; k < chunks; k += W, b ^= 1) {
-                const int s = 2 * w + (int)b;
-                if (!ok(hipEventSynchronize(slots.ev[s]))) return;
-                take(k, slots.at(s));
-                if (ahead < chunks) {
-                    if (!send(ahead, s)) return;
-                    ahead += W;
-                }
+    std::mutex mu;                           // guards what follows
+    int spare[2 * MAX_WORKERS], spares = 0;  // slots not in use
+    struct Sent {
+        int slot;
+        size_t chunk;
+    } sent[2 * MAX_WORKERS];  // slots the device works on, oldest first
+    int head = 0, sents = 0;
+    size_t next = 0;  // first chunk not begun
+    hipError_t err = hipSuccess;
+    // two more slots, for one more worker; one does for the caller
+    auto grow = [&] {
+        hipError_t e = hipSuccess;
+        for (int k = 0; k < 2 && slots.n < 2 * MAX_WORKERS && (size_t)slots.n < chunks; k++) {
+            if ((e = slots.add()) != hipSuccess) {
+                (void)hipGetLastError();
+                break;
             }
-        } else {
-            size_t n = 0;
-            for (size_t k = w; k < chunks; k += W, n++) {
-                const int s = 2 * w + (int)(n & 1);
-                if (n >= 2 && !ok(hipEventSynchronize(slots.ev[s]))) return;
-                take(k, slots.at(s));
-                if (!send(k, s)) return;
-            }
+            std::lock_guard<std::mutex> lock(mu);
+            spare[spares++] = slots.n - 1;
         }
+        return e;
     };
-    run_workers(W, worker);
+    hipError_t e = grow();
+    if (slots.n == 0) return fail(MRLBM_ENOMEM, "pinned staging memory: %s", hipGetErrorString(e));
+    auto step = [&] {
+        std::unique_lock<std::mutex> lock(mu);
+        // begin a chunk if a slot is there for it, which is one not in use or,
+        // upwards, the one that the device is done with first; otherwise,
+        // downwards, finish the oldest
+        const bool begin = next < chunks && (spares || (!DOWN && sents));
+        const bool wait = begin ? !spares : DOWN && sents;
+        if (err != hipSuccess || !(begin || wait)) return false;
+        Sent s{};
+        if (wait) {
+            s = sent[head];
+            head = (head + 1) % (2 * MAX_WORKERS);
+            sents--;
+        } else {
+            s.slot = spare[--spares];
+        }
+        if (begin) s.chunk = next++;
+        lock.unlock();
+        hipError_t r = wait ? hipEventSynchronize(slots.ev[s.slot]) : hipSuccess;
+        if (r == hipSuccess && begin != DOWN) take(s.chunk, slots.mem[s.slot]);
+        if (r == hipSuccess && begin) {
+            r = launch(s.chunk, slots.mem[s.slot]);
+            if (r == hipSuccess) r = hipEventRecord(slots.ev[s.slot], c->stream);
+        }
+        lock.lock();
+        if (r != hipSuccess) err = r;
+        if (begin)
+            sent[(head + sents++) % (2 * MAX_WORKERS)] = s;
+        else
+            spare[spares++] = s.slot;
+        return true;
+    };
+    run_workers(
+        [&] {
+            std::lock_guard<std::mutex> lock(mu);
+            return chunks - next;
+        },
+        [&] { return grow() == hipSuccess; }, [&] { return hipSetDevice(c->p.device) == hipSuccess; }, step);
     // the slots are released below: nothing may still use them
     e = hipStreamSynchronize(c->stream);
-    if (e == hipSuccess) e = (hipError_t)err.load();
+    if (e == hipSuccess) e = err;
     if (e != hipSuccess) return fail(MRLBM_EHIP, "field transfer: %s", hipGetErrorString(e));
     return MRLBM_OK;
 }
@@ -319,21 +353,23 @@ struct Chunks {
 size_t first_bad_density(const double* rho, size_t N) {
     const size_t per = 1u << 17;
     const size_t chunks = (N + per - 1) / per;
-    const int W = workers_for(chunks);
-    std::atomic<size_t> bad{N};
-    run_workers(W, [&](int w) {
-        for (size_t k = w; k < chunks; k += W) {
-            const size_t end = (k + 1) * per < N ? (k + 1) * per : N;
-            bool ok = true;
-            for (size_t j = k * per; j < end; j++) ok &= rho[j] > 0;
-            if (ok) continue;
-            size_t j = k * per;
-            while (rho[j] > 0) j++;
-            size_t cur = bad.load();
-            while (j < cur && !bad.compare_exchange_weak(cur, j)) {
-            }
-            return;  // this worker's later chunks lie higher
+    std::atomic<size_t> bad{N}, next{0};
+    auto yes = [] { return true; };
+    run_workers([&] { return next < chunks ? chunks - next : 0; }, yes, yes, [&] {
+        const size_t k = next++;
+        // ranges are begun in ascending order: behind one with a bad node
+        // there is nothing to find
+        if (k >= chunks || bad < k * per) return false;
+        const size_t end = (k + 1) * per < N ? (k + 1) * per : N;
+        bool ok = true;
+        for (size_t j = k * per; j < end; j++) ok &= rho[j] > 0;
+        if (ok) return true;
+        size_t j = k * per;
+        while (rho[j] > 0) j++;
+        size_t cur = bad.load();
+        while (j < cur && !bad.compare_exchange_weak(cur, j)) {
         }
+        return false;
     });
     return bad.load();
 }

@@ -229,3 +229,42 @@ def test_macroscopic_fields_own_their_memory():
         mrlbm._lib.check(mrlbm._lib.load().mrlbm_read_macroscopic(lat._h, 0.9, one.ctypes.data_as(mrlbm._lib._dp)))
         for f, w in zip(got, one):
             assert np.array_equal(f.reshape(-1, order="F"), w)
+
+
+def test_lowest_bad_density_of_many_ranges():
+    """Densities are checked in ranges of 2^17 nodes by as many threads as
+    have a processor; the node that is reported is the lowest bad one."""
+    shape = (160, 128, 104)  # 17 ranges
+    n = int(np.prod(shape))
+    per = 1 << 17
+    rng = np.random.default_rng(5)
+    rho, u = np.ones(n), np.zeros((3, n))
+    with lattice(shape, {}) as lat:
+        lat.init_uniform()
+        cases = [[n - 1], [per - 1, per], [per, 9 * per + 3], [16 * per, 15 * per + 7, 14 * per + 99],
+                 [3 * per + 100, 4 * per, 5 * per, 3 * per + 99]]
+        cases += [list(rng.integers(0, n, 5)) for _ in range(12)]
+        for at in cases:
+            rho[at] = rng.choice([0.0, -1.0, np.nan], len(at))
+            x, y, z = min(at) % 160, min(at) // 160 % 128, min(at) // (160 * 128)
+            with pytest.raises(mrlbm.MrlbmError, match=rf"\({x},{y},{z}\)"):
+                lat.init_fields(rho, *u)
+            rho[at] = 1.0
+        lat.init_fields(rho, *u)
+        assert lat.reduce_checked() == (0.0, 0.0, 0)
+
+
+@pytest.mark.parametrize("storage", STORES)
+def test_many_chunks_both_ways(storage):
+    """Transfers of up to 130 chunks with helpers joining in between."""
+    shape = (128, 104, 128)
+    n = int(np.prod(shape))
+    with lattice(shape, {}, storage) as lat:
+        m = stored(np.random.default_rng(7).normal(size=(10, n)) * 0.01, storage)
+        for _ in range(3):
+            lat.write_moments(m)
+            assert np.array_equal(lat.moments(), m)
+        rho, *u = lat.macroscopic()
+        assert np.array_equal(rho.reshape(-1, order="F"), m[0] + 1.0)
+        for a in range(3):
+            assert np.array_equal(u[a].reshape(-1, order="F"), m[1 + a] / 3)
