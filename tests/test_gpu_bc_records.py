@@ -64,3 +64,29 @@ def test_batch_of_walls_and_periodic_members(n):
             with make(*s) as alone:
                 alone.step(20)
                 assert np.array_equal(alone.moments(), g)
+
+
+@pytest.mark.parametrize("q", [19, 27])
+def test_first_case_against_the_oracle(q):
+    """Walls on all axes and a moving lid, FP32 moments against the FP64
+    oracle, to the bar of the parity tests."""
+    import _oracle
+    from fields import rel_l2
+
+    shape = (64, 32, 24)
+    types = geometry.classify(shape, (1, 1, 1), None, [(2, +1, 1)])
+    with mrlbm.Lattice(shape, q=q, tau=0.58, walls=(1, 1, 1), force=(2e-5, 0, 0), tile=(8, 8, 8)) as lat:
+        lat.set_bc_velocity(1, (0.05, 0.01, 0.0))
+        lat.set_node_types(types)
+        lat.init_uniform(u=(0.02, 0.0, 0.0))
+        lat.step(25)
+        m = lat.moments()
+    o = _oracle.Oracle(*shape, q=q, tau=0.58, walls=(1, 1, 1), force=(2e-5, 0, 0))
+    o.set_bc_velocity(1, (0.05, 0.01, 0.0))
+    o.set_node_types(types)
+    o.init_uniform(u=(0.02, 0.0, 0.0))
+    o.step(25)
+    assert o.count_nan() == 0
+    e = rel_l2(m, o.moments())
+    print("case", q, e, flush=True)
+    assert max(e.values()) <= 1e-5

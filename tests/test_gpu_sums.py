@@ -148,3 +148,10 @@ def test_threads_read_one_lattice():
         for t in th:
             t.join()
     assert not errors
+
+
+@pytest.mark.parametrize("storage", [mrlbm.STORE_FP32, mrlbm.STORE_FP16, mrlbm.STORE_BF16])
+def test_sums_past_one_round_of_the_grid(storage):
+    """More groups of four nodes than 1024 workgroups of 256 lanes, by a part
+    of a round: the loop, its stride and the fold of 1024 records."""
+    test_sums_equal_numpy((136, 104, 88), storage)
