@@ -516,7 +516,9 @@ int write_taylor_green(mrlbm_ctx* c, double u0, int mode) {
         e = hipGetLastError();
     }
     (void)hipFreeAsync(d, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    // also after a failure: the copy may still read the tables
+    const hipError_t idle = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess) e = idle;
     if (e != hipSuccess) return fail(MRLBM_EHIP, "initial vortex: %s", hipGetErrorString(e));
     return MRLBM_OK;
 }
