@@ -61,11 +61,6 @@ struct mrlbm_ctx {
     float* d_uprev = nullptr;         // velocity of the last residual call (3 x N, block layout), on first use
     int64_t mean_count = 0;
 
-    size_t mom_index(int x, int y, int z, int m) const {
-        const int tile = (x / bx) + ntx * ((y / by) + nty * (z / bz));
-        const int t = (x % bx) + bx * ((y % by) + by * (z % bz));
-        return (size_t)tile * 10 * T + (size_t)m * T + t;
-    }
     size_t node_index(int x, int y, int z) const {
         const int tile = (x / bx) + ntx * ((y / by) + nty * (z / bz));
         const int t = (x % bx) + bx * ((y % by) + by * (z % bz));

@@ -293,9 +293,12 @@ struct LateArgs {
 // With the known masks in scalar registers too (KNOWN_SCALAR below), per
 // step, walls and two spheres: FP16 32^3 7.75 -> 7.04 us, 96x72x80
 // 17.7 -> 16.7, 200x72x104 32.4 -> 30.7, 256x256x128 153.6 -> 146.8,
-// 512x256x256 587 -> 577; BF16 (one chunk still spilled) 200x72x104
-// 32.4 -> 31.0, 512x256x256 589 -> 583. Elsewhere nothing is spilled and the
-// second read only costs (FP32 D3Q19 0.5-2 %).
+// 512x256x256 587 -> 577; BF16 (8x8x8: two floats per lane still spilled)
+// 200x72x104 32.4 -> 31.0, 512x256x256 589 -> 583. Elsewhere nothing is
+// spilled to memory and the second read only costs (FP32 D3Q19 0.5-2 %). The
+// batched kernel of both bodies has its arguments in the instance table, takes
+// fewer scalar registers for them (55 against 70) and reads nothing again; it
+// spills the same two floats for BF16 at 8x8x8 and nothing else.
 template <bool RELOAD>
 __device__ __forceinline__ LateArgs late_args(const StepArgs& first) {
     if constexpr (RELOAD) {
@@ -534,8 +537,9 @@ __device__ __forceinline__ void tile_update(const StepArgs& a, int tile, Lds& L,
 
     // populations leaving the tile (popSave.inc): every node stages its
     // reconstruction terms in LDS, then whole waves evaluate and write the
-    // ghost planes in contiguous runs, each lane only the one population
-    // of its chunk (the other populations of a face node stay unevaluated)
+    // ghost planes in contiguous runs, one window of one face at a time, each
+    // lane the populations of its face node that leave through that face
+    // (halo_store; the others stay unevaluated)
     constexpr int NT = staged_terms<Q>();
     __syncthreads();
     static_for<NT>([&](auto KK) {
@@ -584,9 +588,11 @@ constexpr int step_body_waves() {
 // xcd_grouped gives it), one
 // tile per block: workgroup turnover hides the load latency better than a
 // resident grid walking tiles with a prefetch of the next one (measured on
-// 256^3), and the single-tile body holds fewer scalar registers. For
-// lattices with boundary nodes the library launches the all-bulk tiles and
-// the rest separately.
+// 256^3), and the single-tile body holds fewer scalar registers. It steps
+// lattices without boundary nodes and, all-bulk tiles and the rest launched
+// separately, the shapes with x rows of more than 16 nodes, whose two bodies
+// differ in occupancy; the other shapes take both in one launch
+// (k_step_tile_mixed).
 template <int Q, int BX, int BY, int BZ, bool HAS_BC, int S>
 __global__ __launch_bounds__(BX* BY* BZ) __attribute__((amdgpu_waves_per_eu(step_body_waves<Q, BX, BY, BZ, HAS_BC, S>())))
 void k_step_tile(StepArgs a, const uint32_t* __restrict__ list) {

@@ -10,7 +10,7 @@
 // cross PCIe as FP32 (every stored value is exact in FP32) and are widened
 // to FP64 as they are copied out.
 // Decoding, transposing and index arithmetic on one host thread took
-// 0.95 s for the moments of 256^3 FP32 (1.34 GB as FP64; now 26 ms) and
+// 0.95 s for the moments of 256^3 FP32 (1.34 GB as FP64; now 22 ms) and
 // 1.76 s for the Taylor-Green state (now about a millisecond).
 #include <hip/hip_runtime.h>
 
