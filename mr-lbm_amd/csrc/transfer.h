@@ -41,7 +41,7 @@ inline int transfer_workers(size_t left, unsigned cpus, unsigned running, int ha
 // other programs theirs count too, which only keeps helpers away.
 inline unsigned running_threads() {
     unsigned r = ~0u;
-    FILE* const f = fopen("/proc/loadavg", "r");
+    FILE* const f = fopen("/proc/loadavg", "re");
     if (!f) return r;
     if (fscanf(f, "%*s %*s %*s %u/", &r) != 1) r = ~0u;
     fclose(f);
